@@ -11,6 +11,9 @@ namespace mcke_amd {
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Four floats at any 4-byte address (gfx950 loads and stores 16 bytes per lane at
+// dword alignment).
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int VW> struct VecT;
 template <> struct VecT<1> { using type = float; };
@@ -30,6 +33,16 @@ template <class T> __device__ __forceinline__ T ld_stream(const T* p) {
 }
 template <class T> __device__ __forceinline__ void st_stream(T* p, T v) {
   __builtin_nontemporal_store(v, p);
+}
+// The same for four floats at any 4-byte address.
+__device__ __forceinline__ f32x4 ld_stream4(const float* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(p));
+}
+__device__ __forceinline__ void st_stream4(float* p, f32x4 v) {
+  __builtin_nontemporal_store(static_cast<f32x4_a4>(v), reinterpret_cast<f32x4_a4*>(p));
+}
+__device__ __forceinline__ f32x4 ld4(const float* p) {
+  return *reinterpret_cast<const f32x4_a4*>(p);
 }
 
 // ---------------------------------------------------------------------------
