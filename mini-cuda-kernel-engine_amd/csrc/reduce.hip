@@ -55,50 +55,68 @@ struct SumOp {
   static __device__ __forceinline__ float identity() { return 0.0f; }
   static __device__ __forceinline__ float apply(float a, float b) { return a + b; }
   static __device__ __forceinline__ float wave(float v) { return wave_sum(v); }
+  template <int W> static __device__ __forceinline__ float group(float v) { return wave_sum<W>(v); }
 };
 
 struct MaxOp {
   static __device__ __forceinline__ float identity() { return -INFINITY; }
   static __device__ __forceinline__ float apply(float a, float b) { return fmaxf(a, b); }
   static __device__ __forceinline__ float wave(float v) { return wave_max(v); }
+  template <int W> static __device__ __forceinline__ float group(float v) { return wave_max<W>(v); }
 };
 
 template <class Op> __device__ __forceinline__ float fold4(f32x4 v) {
   return Op::apply(Op::apply(v[0], v[1]), Op::apply(v[2], v[3]));
 }
 
-// Partial of x[begin, end) for this thread, NT lanes striding through it.
-// VEC: begin and end are multiples of 4 and x is 16-byte aligned.
-template <class Op, bool VEC, int U = kLoadUnroll, int NT = kThreads>
-__device__ __forceinline__ float thread_partial(const float* __restrict__ x, int64_t begin,
+// Partial of x[begin, end) for lane t of NT lanes striding through it, float by float.
+template <class Op, int U = kLoadUnroll, int NT = kThreads>
+__device__ __forceinline__ float scalar_partial(const float* __restrict__ x, int64_t begin,
                                                 int64_t end) {
   float acc = Op::identity();
-  if constexpr (VEC) {
-    const f32x4* __restrict__ xv = reinterpret_cast<const f32x4*>(x);
-    const int64_t b4 = begin >> 2, e4 = end >> 2;
-    for (int64_t i = b4 + threadIdx.x; i < e4; i += U * NT) {
-      f32x4 a[U];
+  for (int64_t i = begin + threadIdx.x; i < end; i += U * NT) {
+    float a[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t j = i + u * NT;
-        if (j < e4) a[u] = ld_stream(xv + j);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (i + u * NT < e4) acc = Op::apply(acc, fold4<Op>(a[u]));
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = i + u * NT;
+      if (j < end) a[u] = ld_stream(x + j);
     }
-  } else {
-    for (int64_t i = begin + threadIdx.x; i < end; i += U * NT) {
-      float a[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t j = i + u * NT;
-        if (j < end) a[u] = ld_stream(x + j);
-      }
+    for (int u = 0; u < U; ++u)
+      if (i + u * NT < end) acc = Op::apply(acc, a[u]);
+  }
+  return acc;
+}
+
+// Partial of p[0, n) for lane t of NT lanes striding through it in float4 steps, U loads
+// in flight.  ALIGNED: p is 16-byte aligned and n a multiple of 4.  Otherwise the range
+// is split at its 16-byte boundaries: `head` (0 .. 3) elements, whole vectors, and 0 .. 3
+// elements after them; the up to six edge elements are one float in each of the first
+// lanes (NT >= 8).
+template <class Op, bool ALIGNED, int U, int NT>
+__device__ __forceinline__ float lane_partial(const float* __restrict__ p, int64_t n, int t) {
+  float acc = Op::identity();
+  int64_t head = 0;
+  if constexpr (!ALIGNED) {
+    head = (0 - (reinterpret_cast<uintptr_t>(p) >> 2)) & 3;
+    head = head < n ? head : n;
+  }
+  const int64_t n4 = (n - head) >> 2;
+  const f32x4* __restrict__ xv = reinterpret_cast<const f32x4*>(p + head);
+  if constexpr (!ALIGNED) {
+    const int64_t edges = n - 4 * n4;
+    if (t < edges) acc = Op::apply(acc, ld_stream(p + (t < head ? t : t + 4 * n4)));
+  }
+  for (int64_t i = t; i < n4; i += U * NT) {
+    f32x4 a[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (i + u * NT < end) acc = Op::apply(acc, a[u]);
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = i + u * NT;
+      if (j < n4) a[u] = ld_stream(xv + j);
     }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u * NT < n4) acc = Op::apply(acc, fold4<Op>(a[u]));
   }
   return acc;
 }
@@ -130,16 +148,39 @@ template <class Op> __device__ __forceinline__ float block_combine_tree(float v)
   return buf[0];
 }
 
-template <class Op, bool VEC, bool TREE, bool MEAN>
+template <class Op, bool MEAN>
+__global__ __launch_bounds__(kThreads) void row_reduce_tree_kernel(const float* __restrict__ x,
+                                                                   float* __restrict__ out,
+                                                                   int64_t cols) {
+  const int64_t r = blockIdx.x;
+  float v = scalar_partial<Op>(x + r * cols, 0, cols);
+  v = block_combine_tree<Op>(v);
+  if (threadIdx.x == 0) out[r] = MEAN ? v / static_cast<float>(cols) : v;
+}
+
+template <class Op, bool ALIGNED, bool MEAN>
 __global__ __launch_bounds__(kThreads) void row_reduce_kernel(const float* __restrict__ x,
                                                               float* __restrict__ out,
                                                               int64_t cols) {
   const int64_t r = blockIdx.x;
-  const float* row = x + r * cols;
-  float v = TREE ? thread_partial<Op, false>(row, 0, cols)
-                 : thread_partial<Op, VEC>(row, 0, cols);
-  v = TREE ? block_combine_tree<Op>(v) : block_combine_shfl<Op>(v);
+  float v = lane_partial<Op, ALIGNED, kLoadUnroll, kThreads>(x + r * cols, cols, threadIdx.x);
+  v = block_combine_shfl<Op>(v);
   if (threadIdx.x == 0) out[r] = MEAN ? v / static_cast<float>(cols) : v;
+}
+
+// Short rows: TPR (8 .. 64) consecutive lanes own a row, kThreads / TPR rows per
+// workgroup, combined inside a wave without LDS.
+template <class Op, bool ALIGNED, bool MEAN, int TPR>
+__global__ __launch_bounds__(kThreads) void row_reduce_short_kernel(const float* __restrict__ x,
+                                                                    float* __restrict__ out,
+                                                                    int64_t rows, int64_t cols) {
+  constexpr int kRows = kThreads / TPR;
+  const int t = threadIdx.x % TPR;
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * kRows + threadIdx.x / TPR;
+  if (r >= rows) return;
+  float v = lane_partial<Op, ALIGNED, kLoadUnroll, TPR>(x + r * cols, cols, t);
+  v = Op::template group<TPR>(v);
+  if (t == 0) out[r] = MEAN ? v / static_cast<float>(cols) : v;
 }
 
 // Folds the `split` partials p[0, split) of one row in a fixed order (lane-
@@ -173,7 +214,7 @@ __device__ __forceinline__ float fold_partials(const float* __restrict__ p, int6
 // [s*chunk, min(cols, (s+1)*chunk)) of row r.  With split == 1 the workgroup owns
 // the row and writes out[r]; otherwise it stores its partial to
 // part[r*split + s] for row_reduce_fold_kernel.
-template <class Op, bool VEC, bool MEAN>
+template <class Op, bool ALIGNED, bool MEAN>
 __global__ __launch_bounds__(kSplitThreads) void row_reduce_split_kernel(
     const float* __restrict__ x, float* __restrict__ part, float* __restrict__ out, int64_t cols,
     int64_t chunk, int64_t split) {
@@ -183,7 +224,9 @@ __global__ __launch_bounds__(kSplitThreads) void row_reduce_split_kernel(
   int64_t end = begin + chunk;
   if (end > cols) end = cols;
   float v = Op::identity();
-  if (begin < end) v = thread_partial<Op, VEC, kPass1Unroll, kSplitThreads>(x + r * cols, begin, end);
+  if (begin < end)
+    v = lane_partial<Op, ALIGNED, kPass1Unroll, kSplitThreads>(x + r * cols + begin, end - begin,
+                                                               threadIdx.x);
   v = block_combine_shfl<Op, kSplitThreads>(v);
   if (threadIdx.x != 0) return;
   if (split == 1)
@@ -212,17 +255,38 @@ int64_t two_pass_split(int64_t rows, int64_t cols) {
   return s;
 }
 
+template <class Op, bool MEAN, int TPR>
+int launch_short(const float* x, float* out, int64_t rows, int64_t cols, bool aligned16,
+                 hipStream_t st) {
+  constexpr int kRows = kThreads / TPR;
+  const unsigned g = static_cast<unsigned>((rows + kRows - 1) / kRows);
+  if (aligned16)
+    row_reduce_short_kernel<Op, true, MEAN, TPR><<<g, kThreads, 0, st>>>(x, out, rows, cols);
+  else
+    row_reduce_short_kernel<Op, false, MEAN, TPR><<<g, kThreads, 0, st>>>(x, out, rows, cols);
+  MCKE_LAUNCH_CHECK("row_reduce_short_kernel");
+  return ok();
+}
+
 template <class Op, bool MEAN>
 int launch_one_pass(const float* x, float* out, int64_t rows, int64_t cols, bool tree,
                     hipStream_t st) {
-  const bool vec = (cols % 4 == 0) && aligned(x, 16);
+  const bool aligned16 = (cols % 4 == 0) && aligned(x, 16);
   const unsigned g = static_cast<unsigned>(rows);
-  if (tree)
-    row_reduce_kernel<Op, false, true, MEAN><<<g, kThreads, 0, st>>>(x, out, cols);
-  else if (vec)
-    row_reduce_kernel<Op, true, false, MEAN><<<g, kThreads, 0, st>>>(x, out, cols);
+  if (tree) {
+    row_reduce_tree_kernel<Op, MEAN><<<g, kThreads, 0, st>>>(x, out, cols);
+    MCKE_LAUNCH_CHECK("row_reduce_tree_kernel");
+    return ok();
+  }
+  const int64_t cv = cols / 4;
+  if (cv <= 32) return launch_short<Op, MEAN, 8>(x, out, rows, cols, aligned16, st);
+  if (cv <= 64) return launch_short<Op, MEAN, 16>(x, out, rows, cols, aligned16, st);
+  if (cv <= 128) return launch_short<Op, MEAN, 32>(x, out, rows, cols, aligned16, st);
+  if (cv <= 256) return launch_short<Op, MEAN, 64>(x, out, rows, cols, aligned16, st);
+  if (aligned16)
+    row_reduce_kernel<Op, true, MEAN><<<g, kThreads, 0, st>>>(x, out, cols);
   else
-    row_reduce_kernel<Op, false, false, MEAN><<<g, kThreads, 0, st>>>(x, out, cols);
+    row_reduce_kernel<Op, false, MEAN><<<g, kThreads, 0, st>>>(x, out, cols);
   MCKE_LAUNCH_CHECK("row_reduce_kernel");
   return ok();
 }

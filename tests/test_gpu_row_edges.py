@@ -64,3 +64,64 @@ def test_softmax_width_edges(gpu, orc, cols):
         r = orc.compare(out.get(), want, 1e-5, 1e-6)
         assert r.ok, f"cols={cols} shift={sx},{sy}: {r}"
         del buf
+
+
+REDUCE_COLS = [1, 2, 5, 7, 31, 128, 131, 132, 133, 256, 259, 260, 263, 515, 516, 519, 1027, 1028,
+               1031, 4095, 4099]
+
+
+@pytest.mark.parametrize("cols", REDUCE_COLS)
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_row_reduce_width_edges(gpu, orc, cols, kind):
+    rows = 77
+    x = orc.fill_normal(rows * cols, 0x2ED0 + cols, 0.0, 1.0).reshape(rows, cols)
+    if kind == 1:
+        x[3] = -np.inf
+        x[4, cols // 2] = np.nan if cols > 1 else x[4, 0]
+    x64 = x.astype(np.float64)
+    if kind == 1:
+        want = np.fmax.reduce(x64, axis=1)
+        bar = np.zeros(rows)
+    else:
+        want = x64.sum(axis=1)
+        bar = (cols / 32 + 16) * 2.0 ** -24 * np.abs(x64).sum(axis=1)
+        if kind == 2:
+            want, bar = want / cols, bar / cols + 2.0 ** -24 * np.abs(want / cols)
+    V = gpu.ReduceVariant
+    for sx, _ in SHIFTS[:3]:
+        buf, px = _up(gpu, x, sx)
+        for variant in (V.kWarpShuffle, V.kTwoPass):
+            out = _Out(gpu, rows, 1)
+            if variant == V.kTwoPass:
+                nbytes = gpu.row_reduce_workspace_bytes(rows, cols, variant)
+                ws = gpu.DeviceBuffer(max(4, nbytes))
+                st = gpu.launch_row_reduce_f32(px, out.ptr, rows, cols, kind, variant, ws, nbytes,
+                                               None)
+            else:
+                st = gpu.launch_row_reduce_f32(px, out.ptr, rows, cols, kind, variant)
+            assert st.ok(), str(st)
+            gpu.device_synchronize()
+            got = out.get().astype(np.float64)
+            same = got == want
+            with np.errstate(invalid="ignore"):
+                assert (same | (np.abs(got - want) <= bar)).all(), \
+                    f"cols={cols} kind={kind} {variant!r} shift={sx}"
+        del buf
+
+
+@pytest.mark.parametrize("cols", [100003, 65537])
+def test_split_sum_at_any_alignment(gpu, orc, cols):
+    """The split form's chunks start where the row does, plus a multiple of 4 floats."""
+    rows, V = 3, gpu.ReduceVariant.kTwoPass
+    x = orc.fill_random(rows * cols, 0x5B11 + cols, 0.0, 1.0).reshape(rows, cols)
+    want = x.astype(np.float64).sum(axis=1)
+    nbytes = gpu.row_reduce_workspace_bytes(rows, cols, V)
+    ws = gpu.DeviceBuffer(nbytes)
+    for sx in range(4):
+        buf, px = _up(gpu, x, sx)
+        out = _Out(gpu, rows, 0)
+        st = gpu.launch_row_reduce_f32(px, out.ptr, rows, cols, 0, V, ws, nbytes, None)
+        assert st.ok(), str(st)
+        gpu.device_synchronize()
+        assert np.allclose(out.get(), want, rtol=1e-6, atol=0.0), f"shift={sx}"
+        del buf
