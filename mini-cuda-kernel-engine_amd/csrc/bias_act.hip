@@ -7,14 +7,16 @@
 //     issues 64 x VW x 4 contiguous bytes (1 KiB at VW = 4: a 16-byte
 //     global_load_dwordx4 per lane);
 //   * the bias vector for those columns is loaded once and kept in registers;
-//   * large launches at VW = 4: one one-wave workgroup per 1 KiB strip of a row
+//   * rows that are not whole 1 KiB strips, and VW = 1 and 2: the tensor as one flat
+//     array, one 16-byte vector per lane at any alignment, its columns from a
+//     multiply-shift division;
+//   * large launches of whole strips at VW = 4: one one-wave workgroup per 1 KiB strip of a row
 //     over a flat 1-D grid, so every lane has one 16-byte load in flight, each
 //     wave's life is short (its row and strip come from a multiply-shift
 //     division, no loop), and the hardware streams workgroups through the CUs in
 //     address order;
-//   * narrower widths, launches with a capped grid (max_row_blocks, the
-//     reference's starvation lever) and tensors beyond the flat grid's 32-bit
-//     limits: a 2-D grid of column strips x row blocks that walks rows with a
+//   * launches with a capped grid (max_row_blocks, the reference's starvation
+//     lever) and tensors beyond the flat grids' 32-bit limits: a 2-D grid of column strips x row blocks that walks rows with a
 //     stride of gridDim.y, four per iteration (4 / VW rows per workgroup at once);
 //   * small launches (at most two rounds of resident workgroups at one row each):
 //     256-lane workgroups that each own kChunkRows adjacent rows of their column
@@ -109,6 +111,47 @@ __global__ __launch_bounds__(NT) void bias_act_strip_kernel(const float* __restr
     for (int k = 0; k < VW; ++k) o[k] = act_xb<ACT>(a[k], bv[k]);
   }
   st_stream(reinterpret_cast<V*>(y) + i, o);
+}
+
+// Widths whose rows are not whole 1 KiB strips: the tensor as one flat array, one
+// 16-byte vector per lane and one one-wave workgroup per 1 KiB, whatever the row width
+// and alignment.  A lane's column comes from a multiply-shift division; the vector's
+// other three columns follow it, wrapping to 0 where a row ends inside the vector.  All
+// addresses are 4-byte aligned at least (16-byte ones when x and y are).
+template <int ACT>
+__global__ __launch_bounds__(kRowLanes) void bias_act_flat_kernel(const float* __restrict__ x,
+                                                                  const float* __restrict__ bias,
+                                                                  float* __restrict__ y,
+                                                                  uint32_t n, uint32_t cols,
+                                                                  FastDivU32 by_cols) {
+  const uint32_t v = blockIdx.x * kRowLanes + threadIdx.x;
+  const uint32_t i = 4u * v;
+  if (i >= n) return;
+  const uint32_t col = i - by_cols.div(i) * cols;
+  if (n - i >= 4u) {
+    const f32x4 a = ld_stream4(x + i);
+    f32x4 b;
+    if (col + 4u <= cols) {
+      b = ld4(bias + col);
+    } else {
+      uint32_t c = col;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        b[k] = bias[c];
+        c = c + 1u == cols ? 0u : c + 1u;
+      }
+    }
+    f32x4 o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = act_xb<ACT>(a[k], b[k]);
+    st_stream4(y + i, o);
+    return;
+  }
+  uint32_t c = col;   // the array's last one to three elements
+  for (uint32_t k = i; k < n; ++k) {
+    st_stream(y + k, act_xb<ACT>(ld_stream(x + k), bias[c]));
+    c = c + 1u == cols ? 0u : c + 1u;
+  }
 }
 
 // Small launches: workgroup row blockIdx.y owns R adjacent matrix rows at a time
@@ -245,6 +288,31 @@ template <int VW>
 int launch_fused_vw(const float* x, const float* bias, float* y, int64_t rows, int64_t cols,
                     int act, hipStream_t s, int max_row_blocks) {
   const int64_t cols_v = cols / VW;
+  constexpr int L = kRowBytes / (4 * VW);
+  // The flat array, for rows that do not split into whole 1 KiB strips (the strip and
+  // chunk kernels then leave lanes idle in each row's last one) and for VW = 1 and 2,
+  // where the row kernels move 4 or 8 bytes per load.  GELU_tanh, flat against the
+  // others: 16384 x 4095 (VW = 1) 81.9 vs 103.4 us, 16384 x 4094 (VW = 2) 83.3 vs 99.6,
+  // 16384 x 4100 (VW = 4, strips) 81.6 vs 100.4, 65536 x 64 7.1 vs 16.0, 1000 x 1000
+  // (chunks) 3.2 vs 3.9; with whole strips the others lead: 16384 x 4096 80.7 vs 81.3,
+  // 4096 x 1024 (chunks) 6.6 vs 7.0.  Element numbers stay below 2^31 (FastDivU32).
+  const int64_t n = rows <= INT32_MAX / cols ? rows * cols : int64_t{INT32_MAX} + 1;
+  if (max_row_blocks <= 0 && n <= INT32_MAX && (VW < 4 || cols_v % L != 0)) {
+    const FastDivU32 by = FastDivU32::make(static_cast<uint32_t>(cols));
+    const unsigned g = static_cast<unsigned>(((n + 3) / 4 + kRowLanes - 1) / kRowLanes);
+    const uint32_t n32 = static_cast<uint32_t>(n), c32 = static_cast<uint32_t>(cols);
+#define MCKE_FLAT(A) bias_act_flat_kernel<A><<<g, kRowLanes, 0, s>>>(x, bias, y, n32, c32, by)
+    switch (act) {
+      case kActNone: MCKE_FLAT(kActNone); break;
+      case kActRelu: MCKE_FLAT(kActRelu); break;
+      case kActGeluErf: MCKE_FLAT(kActGeluErf); break;
+      case kActGeluTanh: MCKE_FLAT(kActGeluTanh); break;
+      default: return invalid("launch_bias_act_f32: unknown activation " + std::to_string(act));
+    }
+#undef MCKE_FLAT
+    MCKE_LAUNCH_CHECK("bias_act_flat_kernel");
+    return ok();
+  }
   const int64_t gx = (cols_v + kThreads - 1) / kThreads;
   if (gx * rows <= kChunkMaxBlocks) {
     const dim3 grid = grid_2d(rows, cols_v, max_row_blocks, kThreads, kChunkRows);
@@ -260,7 +328,6 @@ int launch_fused_vw(const float* x, const float* bias, float* y, int64_t rows, i
     MCKE_LAUNCH_CHECK("bias_act_chunk_kernel");
     return ok();
   }
-  constexpr int L = kRowBytes / (4 * VW);
   // The flat grid: rows x strips workgroups of L lanes, within the 32-bit limits
   // of the grid, of the global work size and of FastDivU32's operands.  At VW = 4
   // only: a lane then has a 16-byte load in flight, where at VW = 1 and 2 it would

@@ -125,3 +125,35 @@ def test_split_sum_at_any_alignment(gpu, orc, cols):
         gpu.device_synchronize()
         assert np.allclose(out.get(), want, rtol=1e-6, atol=0.0), f"shift={sx}"
         del buf
+
+
+@pytest.mark.parametrize("act", [0, 1, 2, 3])
+@pytest.mark.parametrize("cols", [1, 2, 3, 5, 63, 100, 129, 252, 255, 257, 260, 1000, 4095])
+def test_bias_act_any_width_matches_the_row_kernel(gpu, orc, cols, act):
+    rows = 301 if cols < 64 else 37
+    x = orc.fill_normal(rows * cols, 0xB1A5 + cols, 0.0, 2.0)
+    x[0], x[-1] = np.inf, -np.inf
+    bias = orc.fill_random(cols, 0xB1A6 + cols, -0.5, 0.5)
+    db, pb = _up(gpu, bias, 0)
+    dx, px = _up(gpu, x, 0)
+    widest = min(gpu.max_vector_width_f32(p, cols) for p in (px, pb))
+    ref = _Out(gpu, rows * cols, 0)
+    st = gpu.launch_bias_act_f32(px, pb, ref.ptr, rows, cols, act, 1, None, rows)
+    assert st.ok(), str(st)
+    gpu.device_synchronize()
+    want = ref.get().view(np.uint32)
+    for vw in (w for w in (1, 2, 4) if w <= widest):
+        out = _Out(gpu, rows * cols, 0)
+        st = gpu.launch_bias_act_f32(px, pb, out.ptr, rows, cols, act, vw)
+        assert st.ok(), str(st)
+        gpu.device_synchronize()
+        assert np.array_equal(out.get().view(np.uint32), want), f"vw={vw}"
+    for sx, sy, sb in ((1, 2, 3), (3, 0, 1)):
+        d2, p2 = _up(gpu, x, sx)
+        b2, q2 = _up(gpu, bias, sb)
+        out = _Out(gpu, rows * cols, sy)
+        st = gpu.launch_bias_act_f32(p2, q2, out.ptr, rows, cols, act, 1)
+        assert st.ok(), str(st)
+        gpu.device_synchronize()
+        assert np.array_equal(out.get().view(np.uint32), want), f"shift={sx},{sy},{sb}"
+    del db, dx
