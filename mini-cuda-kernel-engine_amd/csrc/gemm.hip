@@ -252,6 +252,8 @@ struct MfmaCfg {
   bool even_dma = false;
   // The same three kernels with the fused bias + activation epilogue.
   MfmaFn even_f = nullptr, vec_f = nullptr, scalar_f = nullptr;
+  // The direct-to-LDS kernel's form for any M, N >= bn, K >= 32 and 4-byte alignment.
+  MfmaFn edge = nullptr, edge_f = nullptr;
 };
 
 #define MCKE_MFMA_CFG(BM, BN, BK)                                                     \
@@ -267,7 +269,9 @@ struct MfmaCfg {
    &gemm_mfma_kernel<BM, BN, 32, true, false>, &gemm_mfma_kernel<BM, BN, 32, false, false>, \
    kDmaThreads<BM, BN, KS>, true, &gemm_mfma_dma_kernel<BM, BN, ST, KS, true>,        \
    &gemm_mfma_kernel<BM, BN, 32, true, false, true>,                                  \
-   &gemm_mfma_kernel<BM, BN, 32, false, false, true>}
+   &gemm_mfma_kernel<BM, BN, 32, false, false, true>,                                 \
+   &gemm_mfma_dma_kernel<BM, BN, ST, KS, false, true>,                                \
+   &gemm_mfma_dma_kernel<BM, BN, ST, KS, true, true>}
 
 // 64 x 64 tiles serve small problems, whose single round of tiles leaves one
 // workgroup per CU.  Their direct-to-LDS kernel meets at its barrier in the
@@ -300,6 +304,8 @@ struct Spec {
   MfmaFn mfma_even = nullptr;     // unchecked 16-byte variant for whole tiles
   MfmaFn mfma_f = nullptr;        // the two with the fused bias + activation epilogue
   MfmaFn mfma_even_f = nullptr;
+  MfmaFn mfma_edge = nullptr;     // direct-to-LDS kernel for shapes that are not whole tiles
+  MfmaFn mfma_edge_f = nullptr;
   int even_threads = 0;           // their block size
   bool even_dma = false;          // they take 32-bit per-lane source offsets
   dim3 block{1, 1, 1};
@@ -363,6 +369,8 @@ int gemm_spec(int variant, const mcke_gemm_tile* tile, bool vec4, Spec& s) {
       s.mfma_even = vec4 ? cfg->even : nullptr;
       s.mfma_f = vec4 ? cfg->vec_f : cfg->scalar_f;
       s.mfma_even_f = vec4 ? cfg->even_f : nullptr;
+      s.mfma_edge = cfg->edge;
+      s.mfma_edge_f = cfg->edge_f;
       s.even_threads = cfg->even_threads;
       s.even_dma = cfg->even_dma;
       s.tile_k = cfg->bk;
@@ -419,8 +427,8 @@ int launch_rocblas(const float* a, const float* b, float* c, int m, int n, int k
   return ok();
 }
 
-// One kMfmaF32 launch: whole tiles take the direct-to-LDS kernel, other shapes the
-// staged one; `fused` picks the instantiations with the bias + activation
+// One kMfmaF32 launch: whole tiles take the direct-to-LDS kernel; other shapes its EDGE
+// form where a tile's columns fit in a row of B and K holds a stage, else the staged kernel; `fused` picks the instantiations with the bias + activation
 // epilogue, which route shapes exactly as the plain ones do (so a fused launch
 // accumulates in the plain launch's order).
 int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, const float* b,
@@ -430,12 +438,17 @@ int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, con
   const int64_t tiles_n = (n + sp.tile_n - 1) / sp.tile_n;
   if (tiles_m * tiles_n > 2147483647LL)
     return invalid(std::string(who) + ": too many tiles for one launch");
+  const bool offsets32 = static_cast<int64_t>(sp.tile_m) * k < (int64_t{1} << 30) &&
+                         static_cast<int64_t>(32) * n < (int64_t{1} << 30);
   const bool whole = sp.mfma_even && m % sp.tile_m == 0 && n % sp.tile_n == 0 &&
-                     k % sp.tile_k == 0 &&
-                     (!sp.even_dma || (static_cast<int64_t>(sp.tile_m) * k < (int64_t{1} << 30) &&
-                                       static_cast<int64_t>(32) * n < (int64_t{1} << 30)));
-  MfmaFn fn = whole ? (fused ? sp.mfma_even_f : sp.mfma_even) : (fused ? sp.mfma_f : sp.mfma);
-  const dim3 block = whole ? dim3(static_cast<unsigned>(sp.even_threads), 1, 1) : sp.block;
+                     k % sp.tile_k == 0 && (!sp.even_dma || offsets32);
+  // EDGE loads assume floats at 4-byte addresses.
+  const bool edge = !whole && sp.mfma_edge && n >= sp.tile_n && k >= 32 && offsets32 &&
+                    aligned(a, 4) && aligned(b, 4) && aligned(c, 4) && aligned(epi.bias, 4);
+  MfmaFn fn = fused ? (whole ? sp.mfma_even_f : edge ? sp.mfma_edge_f : sp.mfma_f)
+                    : (whole ? sp.mfma_even : edge ? sp.mfma_edge : sp.mfma);
+  const dim3 block =
+      whole || edge ? dim3(static_cast<unsigned>(sp.even_threads), 1, 1) : sp.block;
   if (tiles_m * tiles_n * static_cast<int64_t>(block.x) > int64_t{UINT32_MAX})
     return invalid(std::string(who) + ": tiles x lanes exceed the grid's 32-bit work size; use a "
                    "larger tile");

@@ -33,6 +33,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 #include <utility>
 
 #include "device_math.hpp"
@@ -412,6 +413,93 @@ __device__ __forceinline__ void mfma_store_c_whole_act(const f32x16 (&acc)[MT][N
   }
 }
 
+// Two or four floats stored at any 4-byte address.
+typedef float f32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+
+// The C store of the direct-to-LDS kernel's EDGE form: rows past M and columns before
+// n_first (another tile's) are left alone, and a lane's 2 or 4 adjacent columns go out as
+// one store at 4-byte alignment unless n_first falls inside them.  The same values as
+// mfma_store_c_whole.  ACT < 0: plain, C = alpha * acc + beta * C; else fused (beta = 0).
+template <int MT, int NT, int ACT>
+__device__ __forceinline__ void mfma_store_c_edge(const f32x16 (&acc)[MT][NT],
+                                                  float* __restrict__ C, int M, int N, int m0,
+                                                  int n0, int n_first, int wm, int wn, int h,
+                                                  int c, float alpha, float beta,
+                                                  const float* __restrict__ bias) {
+  constexpr int WM = 32 * MT, WN = 32 * NT;
+  constexpr int W = NT == 2 ? 2 : 4;    // columns per store
+  const int col = n0 + wn * WN + (NT == 1 ? (c & ~3) : NT * c);
+  float b[W] = {};
+  if constexpr (ACT >= 0) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) b[j] = bias[col + j];
+  }
+  using Q = std::conditional_t<W == 4, f32x4, f32x2>;
+  using QA = std::conditional_t<W == 4, f32x4_a4, f32x2_a4>;
+  auto put = [&](int row, const float (&v)[W]) {
+    if (row >= M) return;
+    float* p = C + static_cast<int64_t>(row) * N + col;
+    // The values before the branch on n_first, so that the accumulators are read once.
+    Q o;
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      if constexpr (ACT >= 0) o[j] = epi_act<(ACT >= 0 ? ACT : 0)>(alpha * v[j], b[j]);
+      else o[j] = alpha * v[j];
+    }
+    if (ACT < 0 && beta != 0.0f) o += beta * static_cast<Q>(*reinterpret_cast<const QA*>(p));
+    if (col >= n_first) {
+      *reinterpret_cast<QA*>(p) = static_cast<QA>(o);
+    } else {
+#pragma unroll
+      for (int j = 1; j < W; ++j)
+        if (col + j >= n_first) p[j] = o[j];
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int row0 = m0 + wm * WM + i * 32 + 4 * h;
+    if constexpr (NT == 1) {
+      const int t = c & 3;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v[4] = {acc[i][0][4 * q], acc[i][0][4 * q + 1], acc[i][0][4 * q + 2],
+                      acc[i][0][4 * q + 3]};
+        quad_transpose(v[0], v[1], v[2], v[3], t);
+        put(row0 + 8 * q + t, v);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float v[W];
+#pragma unroll
+        for (int j = 0; j < W; ++j) v[j] = acc[i][j][r];
+        put(row0 + 8 * (r / 4) + (r % 4), v);
+      }
+    }
+  }
+}
+
+template <int MT, int NT, bool FUSED>
+__device__ __forceinline__ void mfma_epilogue_edge(const f32x16 (&acc)[MT][NT],
+                                                   float* __restrict__ C, int M, int N, int m0,
+                                                   int n0, int n_first, int wm, int wn, int h,
+                                                   int c, float alpha, float beta, EpiArgs epi) {
+  auto store = [&]<int ACT>() {
+    mfma_store_c_edge<MT, NT, ACT>(acc, C, M, N, m0, n0, n_first, wm, wn, h, c, alpha, beta,
+                                   epi.bias);
+  };
+  if constexpr (!FUSED) {
+    store.template operator()<-1>();
+  } else {
+    switch (epi.act) {
+      case kActNone: store.template operator()<kActNone>(); break;
+      case kActRelu: store.template operator()<kActRelu>(); break;
+      case kActGeluErf: store.template operator()<kActGeluErf>(); break;
+      default: store.template operator()<kActGeluTanh>(); break;
+    }
+  }
+}
+
 // The store at a kernel's end: plain, or fused with the activation picked once
 // (a uniform branch around four copies of the store loop).
 template <int MT, int NT, bool VEC, bool WHOLE, bool FUSED>
@@ -665,9 +753,10 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_mfma_kernel(
 
 
 // ---------------------------------------------------------------------------
-// Whole-tile variant with direct-to-LDS loads (gfx950 global_load_lds_dwordx4).
+// Variant with direct-to-LDS loads (gfx950 global_load_lds_dwordx4).
 //
-// For M % BM == N % BN == K % 32 == 0 and 16-byte aligned A and B.  The next
+// For M % BM == N % BN == K % 32 == 0 and 16-byte aligned A and B; the EDGE form (below)
+// takes any M, N >= BN, K >= 32 and 4-byte alignment.  The next
 // stage is fetched straight from global memory into the other LDS buffer: no
 // VGPR staging, no ds_write, and no wait on the loads until the step's closing
 // barrier.  One such instruction writes its 64 lanes' 16 bytes to 1 KB of
@@ -725,7 +814,18 @@ __device__ __forceinline__ void mfma_dma_issue(int a_floats, const uint32_t (&of
 // one wave wide and high, uses it to give its workgroup four waves.  The sum
 // order over K differs from KS = 1 (the groups' partials are added last), and is
 // fixed for a given KS.
-template <int BM, int BN, int STAGES, int KS = 1, bool FUSED = false>
+//
+// EDGE: any M, any N >= BN, any K >= 32, operands at 4-byte alignment (which is all a
+// direct-to-LDS load asks of its source), with the whole-tile loop unchanged:
+//   * rows past M read row M - 1 again and are not stored;
+//   * the last tile column starts at N - BN, so that no load leaves a row of B; the
+//     columns that the tile before it owns are computed again and not stored;
+//   * the K % 32 remainder is the first stage, not the last: its columns [0, K % 32) are
+//     loaded through registers with bounds checks, padded with zeros in both operands,
+//     while the prologue's other stages are in flight, and the whole stages follow.
+// These shapes took the staged kernel before: 3000 x 4096 x 1024 fused GELU 286 us there;
+// 1531 x 1021 x 2053 (4-byte loads) 118 us.
+template <int BM, int BN, int STAGES, int KS = 1, bool FUSED = false, bool EDGE = false>
 __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_kernel(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M,
     int N, int K, float alpha, float beta, int tiles_m, int tiles_n, EpiArgs epi) {
@@ -757,7 +857,9 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
 
   int tm, tn;
   mfma_tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * BM, n_first = tn * BN;
+  const int n0 = EDGE && n_first > N - BN ? N - BN : n_first;
+  const int rem = EDGE ? K % BK : 0;
 
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
@@ -771,14 +873,18 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
   // B per stage), less each instruction's immediate offset.  The launcher keeps
   // BM K and 32 N below 2^30 floats, so they fit 32 bits; row >= 8 ii (A) and
   // (e / BN) N + e % BN >= e >= 256 ii (B, N >= BN) keep them non-negative.
+  // EDGE clamps rows to M - 1, so there the offsets are kept non-negative by 3 KB that the
+  // base gives back.
   const int jr = lane / 8, jp = lane % 8;
+  constexpr uint32_t kBaseA = EDGE ? 3072u : 0u;
   uint32_t offA[NA], offB[NB];
 #pragma unroll
   for (int ii = 0; ii < NA; ++ii) {
     const int ch = wave * NA + ii;
-    const int row = 8 * ch + jr;
-    const int slot = jp ^ jr ^ (ch & 1);          // f(row) = jr ^ (ch & 1)
-    offA[ii] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(K) + 4u * slot) * 4u -
+    const int row_t = 8 * ch + jr;
+    const int row = EDGE && row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
+    const int slot = jp ^ jr ^ (ch & 1);          // f(row_t) = jr ^ (ch & 1)
+    offA[ii] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(K) + 4u * slot) * 4u + kBaseA -
                1024u * (ii % 4);
   }
 #pragma unroll
@@ -787,8 +893,11 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
     offB[ii] = (static_cast<uint32_t>(e / BN) * static_cast<uint32_t>(N) + e % BN) * 4u -
                1024u * (ii % 4);
   }
-  const char* a_base = reinterpret_cast<const char*>(A + static_cast<int64_t>(m0) * K);
-  const char* b_base = reinterpret_cast<const char*>(B + n0);
+  // With a remainder, stage st > 0 holds K columns from BK st - pad on.
+  const int pad = rem ? BK - rem : 0;
+  const char* a_base = reinterpret_cast<const char*>(A) +
+                       (static_cast<int64_t>(m0) * K - pad) * 4 - static_cast<int64_t>(kBaseA);
+  const char* b_base = reinterpret_cast<const char*>(B) + (n0 - static_cast<int64_t>(pad) * N) * 4;
   const int64_t stepB_bytes = static_cast<int64_t>(BK) * N * 4;
   const uint32_t wave_u = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(wave));
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
@@ -802,13 +911,45 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int ksteps = K / BK;
+  const int ksteps = EDGE ? (K + BK - 1) / BK : K / BK;
+  if constexpr (EDGE) {
+    if (rem) {
+      // Stage 0: the remainder's columns, zero past them, in the stage's layout.
+      constexpr int T = kDmaThreads<BM, BN, KS>;
+#pragma unroll 4
+      for (int li = threadIdx.x; li < BM * 8; li += T) {
+        const int row_t = li / 8, p = li % 8;
+        const int row = row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
+        const int k = 4 * (p ^ (row_t & 7) ^ ((row_t >> 3) & 1));
+        const float* src = A + static_cast<int64_t>(m0 + row) * K + k;
+        f32x4 v{0.0f, 0.0f, 0.0f, 0.0f};
+        if (k + 4 <= rem) {
+          v = ld4(src);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 3; ++e)
+            if (k + e < rem) v[e] = src[e];
+        }
+        *reinterpret_cast<f32x4*>(smem + 4 * li) = v;
+      }
+#pragma unroll 4
+      for (int li = threadIdx.x; li < BK * BN / 4; li += T) {
+        const int kr = li / (BN / 4), c4 = li % (BN / 4);
+        f32x4 v{0.0f, 0.0f, 0.0f, 0.0f};
+        if (kr < rem) v = ld4(B + static_cast<int64_t>(kr) * N + n0 + 4 * c4);
+        *reinterpret_cast<f32x4*>(smem + kAFloats + 4 * li) = v;
+      }
+      // The barrier that publishes stage 0 is a bare one.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  }
   // Prologue: stages 0 .. STAGES-2 in flight.  Past the last K step a stage
   // re-fetches the last one into a buffer nobody reads, which keeps the number of
   // loads per stage -- and so the vmcnt arithmetic below -- uniform.
   if (ksteps > 0) {
 #pragma unroll
     for (int st = 0; st < STAGES - 1; ++st) {
+      if (EDGE && st == 0 && rem) continue;
       const int kk = (st < ksteps ? st : ksteps - 1) * BK;
       [&]<int... I>(std::integer_sequence<int, I...>) {
         (mfma_dma_issue<I, NA, NB>(kAFloats, offA, offB, a_base, b_base, stepB_bytes,
@@ -1104,7 +1245,11 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
           for (int r = 0; r < 16; ++r) acc[i][j][r] += smem[slot(g, i, j, r)];
   }
 
-  mfma_epilogue<MT, NT, true, true, FUSED>(acc, C, M, N, m0, n0, wm, wn, h, c, alpha, beta, epi);
+  if constexpr (EDGE)
+    mfma_epilogue_edge<MT, NT, FUSED>(acc, C, M, N, m0, n0, n_first, wm, wn, h, c, alpha, beta,
+                                      epi);
+  else
+    mfma_epilogue<MT, NT, true, true, FUSED>(acc, C, M, N, m0, n0, wm, wn, h, c, alpha, beta, epi);
 }
 
 }  // namespace mcke_amd

@@ -1,0 +1,99 @@
+"""GPU parity of the direct-to-LDS GEMM kernels at shapes that are not whole tiles: one
+row, column or k past or short of a tile and of a K stage, operands and C at every
+4-byte offset from a 16-byte boundary, C between guard floats that must keep their bits.
+
+Bar: float64 on the same inputs with the reference's K-scaled tolerance (tol_gemm,
+abs_tol_gemm); the fused launch bit-equal to the plain one followed by bias + activation.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_row_edges import _Out, _up
+
+pytestmark = pytest.mark.gpu
+
+TILES = [256, 128, 64, 32]
+
+
+def _tile(m, t):
+    return m.GemmTile(t, t, 32, t // 16, t // 16)
+
+
+def _shapes(t):
+    return [(1, t, 32), (t - 1, t + 1, 33), (t + 1, 2 * t - 1, 63), (t, t + 3, 64),
+            (2 * t + 5, t, 95), (3, 2 * t + 2, 129), (t + 7, t + t // 2, 160),
+            (5, t, 31), (5, t - 1, 64)]          # the last two: the staged kernel
+
+
+@pytest.mark.parametrize("t", TILES)
+def test_gemm_f32_tile_edges(gpu, orc, t):
+    V = gpu.GemmVariant.kMfmaF32
+    for M, N, K in _shapes(t):
+        a = orc.fill_random(M * K, 11 + K).reshape(M, K)
+        b = orc.fill_random(K * N, 12 + N).reshape(K, N)
+        c = orc.fill_random(M * N, 13 + M).reshape(M, N)
+        prod = a.astype(np.float64) @ b.astype(np.float64)
+        for sa, sb, sc, alpha, beta in ((0, 0, 0, 1.0, 0.0), (1, 3, 2, -0.5, 1.5)):
+            da, pa = _up(gpu, a, sa)
+            db, pb = _up(gpu, b, sb)
+            out = _Out(gpu, M * N, sc)
+            full = out.buf.download()
+            full[out.at:out.at + M * N] = np.nan if beta == 0.0 else c.ravel()
+            out.buf.upload(full)
+            st = gpu.launch_gemm_f32(pa, pb, out.ptr, M, N, K, alpha, beta, V, _tile(gpu, t))
+            assert st.ok(), str(st)
+            gpu.device_synchronize()
+            want = alpha * prod + beta * c
+            floor = max(1.0, abs(alpha)) * orc.abs_tol_gemm(K) + 2e-7 * abs(beta)
+            r = orc.compare(out.get(), want.ravel(), orc.tol_gemm(K), floor)
+            assert r.ok, f"{M}x{N}x{K} tile={t} shifts={sa},{sb},{sc}: {r}"
+            del da, db
+
+
+@pytest.mark.parametrize("t", TILES)
+@pytest.mark.parametrize("act", [0, 1, 2, 3])
+def test_fused_tile_edges_match_the_pair(gpu, orc, t, act):
+    V = gpu.GemmVariant.kMfmaF32
+    for M, N, K in _shapes(t)[1:6]:
+        a, b = orc.fill_random(M * K, 21 + K), orc.fill_random(K * N, 22 + N)
+        bias = orc.fill_random(N, 23 + M)
+        da, pa = _up(gpu, a, 1)
+        db, pb = _up(gpu, b, 2)
+        dbias, pbias = _up(gpu, bias, 0)
+        c, y, fused = _Out(gpu, M * N, 0), _Out(gpu, M * N, 0), _Out(gpu, M * N, 3)
+        tile = _tile(gpu, t)
+        for st in (gpu.launch_gemm_f32(pa, pb, c.ptr, M, N, K, 0.75, 0.0, V, tile),
+                   gpu.launch_bias_act_f32(c.ptr, pbias, y.ptr, M, N, act, 1),
+                   gpu.launch_gemm_bias_act_f32(pa, pb, pbias, fused.ptr, M, N, K, 0.75, act,
+                                                tile)):
+            assert st.ok(), str(st)
+        gpu.device_synchronize()
+        assert np.array_equal(fused.get().view(np.uint32), y.get().view(np.uint32)), \
+            f"{M}x{N}x{K} tile={t}"
+        del da, db, dbias
+
+
+@pytest.mark.parametrize("t", TILES)
+def test_gemm_remainder_keeps_special_values_apart(gpu, orc, t):
+    """K % 32 != 0 pads both operands with zeros: infinities and NaN in the last columns of
+    A, the last rows of B, and past the operands' ends reach their own outputs only."""
+    M, N, K = t + 1, t + 5, 45
+    a = orc.fill_random(M * K, 31).reshape(M, K)
+    b = orc.fill_random(K * N, 32).reshape(K, N)
+    a[M - 1, 3], a[0, K - 1] = np.nan, np.inf
+    b[K - 1, N - 1] = -np.inf
+    want = np.einsum("mk,kn->mn", a.astype(np.float64), b.astype(np.float64))
+    da, pa = _up(gpu, a, 0)
+    db, pb = _up(gpu, b, 0)
+    out = _Out(gpu, M * N, 0)
+    st = gpu.launch_gemm_f32(pa, pb, out.ptr, M, N, K, 1.0, 0.0, gpu.GemmVariant.kMfmaF32,
+                             _tile(gpu, t))
+    assert st.ok(), str(st)
+    gpu.device_synchronize()
+    got = out.get().reshape(M, N)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fin = np.isfinite(want)
+    assert orc.compare(got[fin], want[fin], orc.tol_gemm(K), orc.abs_tol_gemm(K)).ok
