@@ -24,6 +24,7 @@
 #include "common.hpp"
 #include "device_math.hpp"
 #include "gemm_mfma.hpp"
+#include "gemm_rows.hpp"
 
 namespace mcke_amd {
 namespace {
@@ -427,13 +428,49 @@ int launch_rocblas(const float* a, const float* b, float* c, int m, int n, int k
   return ok();
 }
 
-// One kMfmaF32 launch: whole tiles take the direct-to-LDS kernel; other shapes its EDGE
-// form where a tile's columns fit in a row of B and K holds a stage, else the staged kernel; `fused` picks the instantiations with the bias + activation
-// epilogue, which route shapes exactly as the plain ones do (so a fused launch
-// accumulates in the plain launch's order).
+using RowsFn = void (*)(const float*, const float*, float*, int, int, int, float, float, EpiArgs);
+
+// The few-rows kernel for a 32 x 32 tile launch, if it is the better one, and its column
+// width: the narrowest of 16, 32 and 64 columns a workgroup whose workgroups are all
+// resident at once.  Wider ones, or more row blocks than two, pay off from K = 1024 on
+// (7 x 6015 x 628: 7.4 against 7.3 us for the tile; 64 x 4096 x 256: 5.0 against 4.4;
+// 32 x 8192 x 1024: 9.4 against 10.4).  Past 64 rows the product is bound by the MFMAs.
+// Per-lane source offsets are 32-bit.
+RowsFn find_rows(int64_t m, int64_t n, int64_t k, bool fused, int* width) {
+  if (m > 64 || n < 16 || k < 1 || 64 * k >= (int64_t{1} << 30)) return nullptr;
+  const int64_t cus = device_cu_count();
+  const int nw = (n + 15) / 16 <= cus ? 1 : (n + 31) / 32 <= cus ? 2 : 4;
+  if ((n + 16 * nw - 1) / (16 * nw) > cus) return nullptr;
+  const int mt = m <= 16 ? 1 : m <= 32 ? 2 : 4;
+  if ((nw > 1 || mt > 2) && k < 1024) return nullptr;
+  *width = 16 * nw;
+#define MCKE_ROWS(MT, NW) \
+  if (mt == MT && nw == NW) \
+    return fused ? &gemm_rows_kernel<MT, NW, true> : &gemm_rows_kernel<MT, NW, false>;
+  MCKE_ROWS(1, 1) MCKE_ROWS(1, 2) MCKE_ROWS(1, 4)
+  MCKE_ROWS(2, 1) MCKE_ROWS(2, 2) MCKE_ROWS(4, 1)
+#undef MCKE_ROWS
+  return nullptr;   // more rows at wider columns: the tile
+}
+
+// One kMfmaF32 launch: few rows at the 32 x 32 tile take the few-rows kernel, whole tiles
+// the direct-to-LDS kernel, and other shapes its EDGE form where a tile's columns fit in a
+// row of B and K holds a stage, else the staged kernel; `fused` picks the instantiations
+// with the bias + activation epilogue, which route shapes exactly as the plain ones do
+// (so a fused launch accumulates in the plain launch's order).
 int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, const float* b,
                 float* c, int64_t m, int64_t n, int64_t k, float alpha, float beta, EpiArgs epi,
                 hipStream_t s) {
+  // The kernels below load and store floats at 4-byte addresses.
+  const bool floats = aligned(a, 4) && aligned(b, 4) && aligned(c, 4) && aligned(epi.bias, 4);
+  int width = 0;
+  const RowsFn rows_fn = sp.tile_m == 32 && floats ? find_rows(m, n, k, fused, &width) : nullptr;
+  if (rows_fn) {
+    rows_fn<<<static_cast<unsigned>((n + width - 1) / width), kRowsThreads, 0, s>>>(
+        a, b, c, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), alpha, beta, epi);
+    MCKE_LAUNCH_CHECK(fused ? "gemm_rows_kernel (bias + activation)" : "gemm_rows_kernel");
+    return ok();
+  }
   const int64_t tiles_m = (m + sp.tile_m - 1) / sp.tile_m;
   const int64_t tiles_n = (n + sp.tile_n - 1) / sp.tile_n;
   if (tiles_m * tiles_n > 2147483647LL)
@@ -442,9 +479,7 @@ int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, con
                          static_cast<int64_t>(32) * n < (int64_t{1} << 30);
   const bool whole = sp.mfma_even && m % sp.tile_m == 0 && n % sp.tile_n == 0 &&
                      k % sp.tile_k == 0 && (!sp.even_dma || offsets32);
-  // EDGE loads assume floats at 4-byte addresses.
-  const bool edge = !whole && sp.mfma_edge && n >= sp.tile_n && k >= 32 && offsets32 &&
-                    aligned(a, 4) && aligned(b, 4) && aligned(c, 4) && aligned(epi.bias, 4);
+  const bool edge = !whole && sp.mfma_edge && n >= sp.tile_n && k >= 32 && offsets32 && floats;
   MfmaFn fn = fused ? (whole ? sp.mfma_even_f : edge ? sp.mfma_edge_f : sp.mfma_f)
                     : (whole ? sp.mfma_even : edge ? sp.mfma_edge : sp.mfma);
   const dim3 block =

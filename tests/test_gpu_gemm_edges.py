@@ -97,3 +97,65 @@ def test_gemm_remainder_keeps_special_values_apart(gpu, orc, t):
     assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     fin = np.isfinite(want)
     assert orc.compare(got[fin], want[fin], orc.tol_gemm(K), orc.abs_tol_gemm(K)).ok
+
+
+# (M, N, K) around the few-rows kernel's row blocks (16, 32, 64), column widths (16 up to
+# 4096 columns, 32 and 64 past 4096 and 8192 from K = 1024 on), K chunks (32, dealt to 8
+# waves) and its limits (65 rows, 15 columns: the tile kernels).
+ROWS_SHAPES = [(1, 16, 1), (16, 17, 31), (17, 31, 32), (31, 33, 33), (32, 100, 255), (33, 64, 1024),
+               (48, 77, 1031), (64, 259, 1056), (15, 4095, 257), (16, 4096, 256), (5, 4097, 1024),
+               (16, 4128, 1027), (32, 8192, 1025), (3, 8193, 1055), (16, 16383, 1024),
+               (65, 40, 300), (7, 15, 90)]
+
+
+@pytest.mark.parametrize("shape", ROWS_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_few_rows(gpu, orc, shape):
+    M, N, K = shape
+    V = gpu.GemmVariant.kMfmaF32
+    tile = _tile(gpu, 32)
+    a = orc.fill_random(M * K, 41 + K).reshape(M, K)
+    b = orc.fill_random(K * N, 42 + N).reshape(K, N)
+    c = orc.fill_random(M * N, 43 + M).reshape(M, N)
+    bias = orc.fill_random(N, 44)
+    prod = a.astype(np.float64) @ b.astype(np.float64)
+    rel, floor = orc.tol_gemm(K), orc.abs_tol_gemm(K) + 4e-7
+    for sa, sb, sc, beta in ((0, 0, 0, 0.0), (1, 3, 2, 1.5)):
+        da, pa = _up(gpu, a, sa)
+        db, pb = _up(gpu, b, sb)
+        out = _Out(gpu, M * N, sc)
+        full = out.buf.download()
+        full[out.at:out.at + M * N] = np.nan if beta == 0.0 else c.ravel()
+        out.buf.upload(full)
+        st = gpu.launch_gemm_f32(pa, pb, out.ptr, M, N, K, 0.75, beta, V, tile)
+        assert st.ok(), str(st)
+        gpu.device_synchronize()
+        got = out.get()
+        r = orc.compare(got, (0.75 * prod + beta * c).ravel(), rel, floor)
+        assert r.ok, f"shifts={sa},{sb},{sc}: {r}"
+        if beta == 0.0:
+            # The fused launch has the bits of the pair.
+            dbias, pbias = _up(gpu, bias, 0)
+            y, fused = _Out(gpu, M * N, 0), _Out(gpu, M * N, 1)
+            for st in (gpu.launch_bias_act_f32(out.ptr, pbias, y.ptr, M, N, 3, 1),
+                       gpu.launch_gemm_bias_act_f32(pa, pb, pbias, fused.ptr, M, N, K, 0.75, 3,
+                                                    tile)):
+                assert st.ok(), str(st)
+            gpu.device_synchronize()
+            assert np.array_equal(fused.get().view(np.uint32), y.get().view(np.uint32))
+        del da, db
+
+
+def test_few_rows_repeat_their_bits(gpu, orc):
+    """The same bits on every run (no state between launches)."""
+    M, N, K = 16, 1000, 1003
+    a, b = orc.fill_random(M * K, 51), orc.fill_random(K * N, 52)
+    da, db = gpu.DeviceBuffer.from_array(a), gpu.DeviceBuffer.from_array(b)
+    seen = []
+    for _ in range(3):
+        out = _Out(gpu, M * N, 0)
+        st = gpu.launch_gemm_f32(da, db, out.ptr, M, N, K, 1.0, 0.0, gpu.GemmVariant.kMfmaF32,
+                                 _tile(gpu, 32))
+        assert st.ok(), str(st)
+        gpu.device_synchronize()
+        seen.append(out.get().view(np.uint32).copy())
+    assert np.array_equal(seen[0], seen[1]) and np.array_equal(seen[0], seen[2])
