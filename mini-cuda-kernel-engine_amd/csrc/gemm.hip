@@ -612,36 +612,37 @@ int mcke_launch_gemm_lp_vendor(const void* a, const void* b, void* c, int ab_dty
 
 int mcke_gemm_mfma_default_tile(int64_t m, int64_t n, int64_t k, mcke_gemm_tile* out) {
   if (!out) return invalid("gemm_mfma_default_tile: null out");
-  (void)k;
-  // What decides is how evenly a tile size fills whole rounds of CUs: a launch
-  // takes as long as its busiest CU, so a partial last round costs a full one.
-  // Each candidate is scored by its sustained rate with every CU busy, times the
-  // share of its rounds' tile area that is useful work (m*n over rounds * CUs *
-  // tile area: partial rounds and the padding of edge tiles both count against
-  // it); the best score wins (ties: larger tile).
-  // Rates measured on MI355X (gfx950, 256 CUs), fp32, whole-tile shapes: 256 x 256
-  // (one workgroup per CU) ~145, 128 x 128 (two per CU) ~137, 64 x 64 ~135, 32 x 32
-  // (four wave groups) ~100 TFLOP/s.  The scores pick the measured winner at every shape timed:
-  // 8192^3 and 8192 x 8192 x {512..2048} -> 256; 4096^3 -> 256 (140 vs 131);
-  // 6144^3 -> 128 (137 vs 107 for 256, 2.25 rounds); 2048^3 and 2048 x 2048 x
-  // 8192 -> 128 (125 vs 120 for 64); 3072^3 -> 64 (125 vs 101); 1024^3 -> 64
-  // (103 vs 85 for 32); 512^3 -> 32 (40 vs 23 for 64); 256^3 -> 32.
-  // Short K costs every tile alike (measured down to K = 512), so K is not weighed.
-  struct Cand { int t; double rate; mcke_gemm_tile tile; };
-  static const Cand cands[] = {{256, 145.0, {256, 256, 32, 16, 16}},
-                               {128, 137.0, {128, 128, 32, 8, 8}},
-                               {64, 135.0, {64, 64, 32, 4, 4}},
-                               {32, 100.0, {32, 32, 32, 2, 2}}};
+  // What decides is how evenly a tile size fills the CUs: a launch takes as long as its
+  // busiest CU, which runs r = ceil(tiles / CUs) tiles.  Each candidate's cost is that
+  // CU's time, in us per 4096 of K, from launches timed on MI355X (gfx950, 256 CUs), and
+  // the lowest one wins (ties: the larger tile).  K itself scales all alike (measured
+  // down to K = 128).
+  //   32:  26 alone on its CU, then 18.4 r (16 x 4096: 25.7; 480 x 816: 37 at r = 2;
+  //        1000 x 1024: 73 at r = 4; 2602 x 1960: 364 at r = 20).
+  //   64:  73 alone, then 64.5 r (1024 x 1024: 75; 1531 x 1021: 132 at r = 2; 1000 x 4096:
+  //        261 at r = 4; 3000 x 4096: 788 at r = 12).
+  //   128: 257 alone, then 240 r, two tiles at a time: an odd last one shares its CU with
+  //        nothing, or falls to a CU that has two (r = 3: 755 .. 949, so r + 0.6).
+  //        2048 x 2048: 257 .. 269, 2048 x 4096: 511, 4096 x 4096 : 956.
+  //   256: 950 r, one at a time (4096 x 4096: 926 .. 974).
+  // Shapes that are not whole tiles cost the two large tiles 3% more (the EDGE form's
+  // row and column checks: 1000 x 4096 x 1024 69.8 us against 68.0 for 1024 rows).
+  struct Cand { int t; double alone, each; mcke_gemm_tile tile; };
+  static const Cand cands[] = {{256, 950.0, 950.0, {256, 256, 32, 16, 16}},
+                               {128, 257.0, 240.0, {128, 128, 32, 8, 8}},
+                               {64, 73.0, 64.5, {64, 64, 32, 4, 4}},
+                               {32, 26.0, 18.4, {32, 32, 32, 2, 2}}};
   const int64_t cus = device_cu_count();
-  double best = -1.0;
+  double best = 0.0;
   for (const Cand& c : cands) {
     const int64_t tiles = ((m + c.t - 1) / c.t) * ((n + c.t - 1) / c.t);
-    const int64_t rounds = (tiles + cus - 1) / cus;
-    const double area = static_cast<double>(rounds * cus) * c.t * c.t;
-    const double score = rounds > 0 ? c.rate * static_cast<double>(m) * static_cast<double>(n) / area
-                                    : 0.0;
-    if (score > best) {
-      best = score;
+    const int64_t r = tiles > 0 ? (tiles + cus - 1) / cus : 1;
+    double cost = c.each * static_cast<double>(r);
+    if (r == 1) cost = c.alone;
+    else if (c.t == 128 && r % 2 == 1) cost += 0.6 * c.each;
+    if (c.t >= 128 && (m % c.t != 0 || n % c.t != 0 || k % 32 != 0)) cost *= 1.03;
+    if (c.t == 256 || cost < best) {
+      best = cost;
       *out = c.tile;
     }
   }
