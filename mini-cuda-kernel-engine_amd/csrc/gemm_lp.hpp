@@ -718,8 +718,11 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma_kernel(
     }(std::make_integer_sequence<int, S::kMfmas>{});
   }
   // No LDS DMA may still be landing, and no LDS read outstanding, when the
-  // workgroup retires.
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  // workgroup retires.  The last step's reads go unused, but they land in these
+  // registers: named in the wait, none of them can hold anything else before it.
+  lds_wait<MT, NT>(av0, bv0);
+  lds_wait<MT, NT>(av1, bv1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   using O = LpOut<OutT>;
   if constexpr (!TRANS) {
@@ -1193,6 +1196,14 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
     step.template operator()<0>(ks);
     step.template operator()<1>(ks + 1);
   }
+  // No LDS DMA may still be landing, and no LDS read outstanding, when the
+  // workgroup retires.  The last step's reads go unused, but they land in these
+  // registers: named after the wait, none of them can hold anything else before it.
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  touch_a<0, MT>(av[0]);
+  touch_a<0, MT>(av[1]);
+  touch_b<0, NT>(bv[0]);
+  touch_b<0, NT>(bv[1]);
   // The accumulators stay in the accumulation registers past the loop: left to
   // itself the compiler copies all of them out at once where the loop and the
   // K == 0 path meet, more than the other register file holds.
@@ -1203,9 +1214,6 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
   // acc_get is inline asm, which the hazard checks do not see into: the last
   // MFMA's results are ready well before these 16 cycles are over.
   asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");
-  // No LDS DMA may still be landing, and no LDS read outstanding, when the
-  // workgroup retires.
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 
   using O = LpOut<OutT>;
   if constexpr (!TRANS) {
