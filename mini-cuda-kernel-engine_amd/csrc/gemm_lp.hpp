@@ -1197,13 +1197,11 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
     step.template operator()<1>(ks + 1);
   }
   // No LDS DMA may still be landing, and no LDS read outstanding, when the
-  // workgroup retires.  The last step's reads go unused, but they land in these
-  // registers: named after the wait, none of them can hold anything else before it.
+  // workgroup retires.  The last step's reads go unused, but they land in register set
+  // 0: named after the wait, it can hold nothing else before it.
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   touch_a<0, MT>(av[0]);
-  touch_a<0, MT>(av[1]);
   touch_b<0, NT>(bv[0]);
-  touch_b<0, NT>(bv[1]);
   // The accumulators stay in the accumulation registers past the loop: left to
   // itself the compiler copies all of them out at once where the loop and the
   // K == 0 path meet, more than the other register file holds.
