@@ -11,79 +11,152 @@
 
 #include "common.hpp"
 #include "gemm_lp.hpp"
+#include "gemm_lp_split.hpp"
 
 namespace mcke_amd {
 namespace {
 
 using LpKernel = const void*;
 
-// LDS stages of the direct-to-LDS kernel per tile (32 KiB per stage at 256 x 256).
-template <int BM, int BN> struct LpDmaStages { static constexpr int value = 4; };
+// Direct-to-LDS 16x16x32 kernel for a BM x BN tile: whole tiles with 16-byte aligned
+// operands and K % 64 == 0, or the EDGE form.  Its per-lane source offsets are 32-bit: BM
+// rows of A and 64 rows of B must span less than 4 GiB.
+template <int BM, int BN>
+bool dma_offsets32(int n, int k) {
+  return static_cast<int64_t>(BM) * k * 2 + 4096 < (int64_t{1} << 32) &&
+         static_cast<int64_t>(64) * n * 2 < (int64_t{1} << 32);
+}
+
+int64_t tile_count(int m, int n, int bm, int bn) {
+  return ((static_cast<int64_t>(m) + bm - 1) / bm) * ((static_cast<int64_t>(n) + bn - 1) / bn);
+}
+
+struct LpArgs {
+  const uint16_t* a;
+  const uint16_t* b;
+  void* c;
+  int m, n, k;
+  float alpha, beta;
+  hipStream_t s;
+};
+
+int check_grid(int64_t tiles, int threads) {
+  if (tiles * threads > int64_t{UINT32_MAX})
+    return invalid("launch_gemm_lp: tiles x lanes exceed the grid's 32-bit work size; use a "
+                   "larger tile");
+  return ok();
+}
+
+template <typename T, typename OutT, int BM, int BN, bool EDGE>
+int launch_dma(const LpArgs& x) {
+  const int64_t tiles = tile_count(x.m, x.n, BM, BN);
+  if (int rc = check_grid(tiles, kMfmaThreads)) return rc;
+  gemm_lp_dma16_kernel<T, OutT, BM, BN, EDGE>
+      <<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
+          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + BM - 1) / BM,
+          (x.n + BN - 1) / BN);
+  MCKE_LAUNCH_CHECK("gemm_lp_dma16_kernel");
+  return ok();
+}
+
+template <typename T, typename OutT, int MT, int NW, int WV>
+int launch_split_as(const LpArgs& x) {
+  constexpr int TM = 16 * MT, TN = 16 * NW;
+  const int64_t tiles = tile_count(x.m, x.n, TM, TN);
+  if (int rc = check_grid(tiles, WV * kWave)) return rc;
+  gemm_lp_split_kernel<T, OutT, MT, NW, WV, 1>
+      <<<static_cast<unsigned>(tiles), WV * kWave, 0, x.s>>>(
+          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + TM - 1) / TM,
+          (x.n + TN - 1) / TN);
+  MCKE_LAUNCH_CHECK("gemm_lp_split_kernel");
+  return ok();
+}
+
+// The split-K kernel by shape.  Few rows over up to 8192 columns: 32 columns a workgroup
+// and 8 waves, for as many workgroups as there are (16 x 4096 x 4096: 16 x 32 11.9 us,
+// 32 x 64 16.1, 64 x 64 18.9; 16 x 16384 x 4096: 38.5, 27.1, 29.0).  Else 32 x 64 up to
+// four tiles per CU (64 x 4096 x 4096: 16.7 us against 21.3 for 64 x 64; 1628 x 800 x 1109:
+// 18.2 against 20.3), 64 x 64 past that (1531 x 4096 x 1024: 34.0 against 40.3;
+// 4032 x 843 x 2744: 70.2 against 86.1).  Widths of 32 .. 63 take 32 columns.
+template <typename T, typename OutT>
+int launch_split(const LpArgs& x) {
+  if (x.n < 64 || (x.m <= 32 && x.n <= 8192))
+    return x.m <= 16 ? launch_split_as<T, OutT, 1, 2, 8>(x) : launch_split_as<T, OutT, 2, 2, 8>(x);
+  if (tile_count(x.m, x.n, 32, 64) <= 1024) return launch_split_as<T, OutT, 2, 4, 4>(x);
+  return launch_split_as<T, OutT, 4, 4, 4>(x);
+}
+
+// The register-staged kernel at the requested tile: what is narrower than any other
+// kernel's tile, or past their 32-bit offsets or grids.
+template <typename T, typename OutT, int BM, int BN>
+int launch_staged(const LpArgs& x, bool vec) {
+  const int64_t tiles = tile_count(x.m, x.n, BM, BN);
+  if (int rc = check_grid(tiles, kMfmaThreads)) return rc;
+  auto* fn = vec ? &gemm_lp_kernel<T, OutT, BM, BN, true, false>
+                 : &gemm_lp_kernel<T, OutT, BM, BN, false, false>;
+  fn<<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
+      x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + BM - 1) / BM,
+      (x.n + BN - 1) / BN);
+  MCKE_LAUNCH_CHECK("gemm_lp_kernel");
+  return ok();
+}
+
+template <typename T, typename OutT, int BM, int BN>
+int launch_dma32(const LpArgs& x) {
+  constexpr int kStages = 4;
+  const int64_t tiles = tile_count(x.m, x.n, BM, BN);
+  if (int rc = check_grid(tiles, kMfmaThreads)) return rc;
+  gemm_lp_dma_kernel<T, OutT, BM, BN, kStages>
+      <<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
+          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, x.m / BM, x.n / BN);
+  MCKE_LAUNCH_CHECK("gemm_lp_dma_kernel");
+  return ok();
+}
+
+// The EDGE form at BM x BN, where the shape and the addresses allow it.
+template <int BM, int BN> bool edge_fits(const LpArgs& x) {
+  return x.n >= BN && x.k >= 64 && x.n % 2 == 0 && x.k % 2 == 0 && aligned(x.a, 4) &&
+         aligned(x.b, 4) && aligned(x.c, 4) && dma_offsets32<BM, BN>(x.n, x.k);
+}
 
 template <typename T, typename OutT, int BM, int BN>
 struct LpTile {
-  // Whole tiles with 16-byte aligned operands take a direct-to-LDS kernel (tiles
-  // with BN >= 128), whose per-lane source offsets are 32-bit: BM rows of A and 32
-  // rows of B must span less than 4 GiB.  K % 64 == 0 takes the 16x16x32 kernel,
-  // the other multiples of 32 the 32x32x16 one.
-  static bool use_dma(bool vec, int m, int n, int k) {
-    if constexpr (BN < 128) {
-      return false;
-    } else {
-      return vec && m % BM == 0 && n % BN == 0 && k % LpDmaShape<BM, BN, 4>::BK == 0 &&
-             static_cast<int64_t>(BM) * k * 2 < (int64_t{1} << 32) &&
-             static_cast<int64_t>(32) * n * 2 < (int64_t{1} << 32);
-    }
-  }
-  static bool use_dma16(int k) { return k % 64 == 0; }
-
-  static int launch(const void* a, const void* b, void* c, int m, int n, int k, float alpha,
-                    float beta, bool vec, hipStream_t s) {
-    const int64_t tiles_m = (static_cast<int64_t>(m) + BM - 1) / BM;
-    const int64_t tiles_n = (static_cast<int64_t>(n) + BN - 1) / BN;
-    if (tiles_m * tiles_n * kMfmaThreads > int64_t{UINT32_MAX})
-      return invalid("launch_gemm_lp: tiles x lanes exceed the grid's 32-bit work size; use a "
-                     "larger tile");
-    const bool even = vec && m % BM == 0 && n % BN == 0 && k % kLpBK == 0;
-    const auto* A = static_cast<const uint16_t*>(a);
-    const auto* B = static_cast<const uint16_t*>(b);
-    auto* C = static_cast<OutT*>(c);
-    const dim3 grid(static_cast<unsigned>(tiles_m * tiles_n)), block(kMfmaThreads);
-    const int tmi = static_cast<int>(tiles_m), tni = static_cast<int>(tiles_n);
+  // Whole tiles run the requested tile's direct-to-LDS kernel (tiles of 128 and more).
+  // Other shapes run its EDGE form, at 128 x 128 from 80 such tiles on and at 256 x 256
+  // where they nearly fill the CUs (fp16 to fp32: 2757 x 432 x 6080, 88 tiles of 128,
+  // 49.9 us against 54.9 for split K; 1628 x 800 x 1110, 91 tiles, 17.2 against 18.2;
+  // 300 x 520 x 1032, 15 tiles, 15.4 against 6; 4095 x 4094 x 4090, 256 tiles of 256,
+  // 130 us against 205 at 128), and otherwise the split-K kernel, which every 64 x 64
+  // launch takes.
+  static int launch(const LpArgs& x, bool vec) {
     if constexpr (BN >= 128) {
-      if (use_dma(vec, m, n, k)) {
-        if (use_dma16(k)) {
-          gemm_lp_dma16_kernel<T, OutT, BM, BN>
-              <<<grid, block, 0, s>>>(A, B, C, m, n, k, alpha, beta, tmi, tni);
-          MCKE_LAUNCH_CHECK("gemm_lp_dma16_kernel");
-        } else {
-          gemm_lp_dma_kernel<T, OutT, BM, BN, LpDmaStages<BM, BN>::value>
-              <<<grid, block, 0, s>>>(A, B, C, m, n, k, alpha, beta, tmi, tni);
-          MCKE_LAUNCH_CHECK("gemm_lp_dma_kernel");
-        }
-        return ok();
-      }
+      if (vec && x.m % BM == 0 && x.n % BN == 0 && x.k % 64 == 0 && x.k > 0 &&
+          dma_offsets32<BM, BN>(x.n, x.k))
+        return launch_dma<T, OutT, BM, BN, false>(x);
+      if constexpr (BM == 128)
+        if (vec && x.m % BM == 0 && x.n % BN == 0 && x.k % 64 == 32 &&
+            tile_count(x.m, x.n, BM, BN) >= 80 && dma_offsets32<BM, BN>(x.n, x.k))
+          return launch_dma32<T, OutT, BM, BN>(x);
+      if constexpr (BM == 256)
+        if (edge_fits<256, 256>(x) && tile_count(x.m, x.n, 256, 256) >= 192)
+          return launch_dma<T, OutT, 256, 256, true>(x);
+      if (edge_fits<128, 128>(x) && tile_count(x.m, x.n, 128, 128) >= 80)
+        return launch_dma<T, OutT, 128, 128, true>(x);
     }
-    if (even)
-      gemm_lp_kernel<T, OutT, BM, BN, true, true>
-          <<<grid, block, 0, s>>>(A, B, C, m, n, k, alpha, beta, tmi, tni);
-    else if (vec)
-      gemm_lp_kernel<T, OutT, BM, BN, true, false>
-          <<<grid, block, 0, s>>>(A, B, C, m, n, k, alpha, beta, tmi, tni);
-    else
-      gemm_lp_kernel<T, OutT, BM, BN, false, false>
-          <<<grid, block, 0, s>>>(A, B, C, m, n, k, alpha, beta, tmi, tni);
-    MCKE_LAUNCH_CHECK("gemm_lp_kernel");
-    return ok();
+    // 16-bit values at 2-byte addresses, per-lane offsets below 4 GiB, and a grid that holds
+    // 32 x 32 tiles of 512 lanes.
+    if (x.n >= 32 && x.k > 0 && tile_count(x.m, x.n, 32, 32) <= int64_t{UINT32_MAX} / 512 &&
+        aligned(x.a, 2) && aligned(x.b, 2) && aligned(x.c, sizeof(OutT)) && static_cast<int64_t>(64) * x.k * 2 < (int64_t{1} << 32) &&
+        static_cast<int64_t>(64) * x.n * 2 < (int64_t{1} << 32))
+      return launch_split<T, OutT>(x);
+    return launch_staged<T, OutT, BM, BN>(x, vec);
   }
   // The instantiation whole-tile shapes run, for attribute queries.
   static LpKernel kernel() {
-    using Fn = void (*)(const uint16_t*, const uint16_t*, OutT*, int, int, int, float, float, int,
-                        int);
-    Fn fn;
-    if constexpr (BN >= 128) fn = &gemm_lp_dma16_kernel<T, OutT, BM, BN>;
-    else fn = &gemm_lp_kernel<T, OutT, BM, BN, true, true>;
-    return reinterpret_cast<LpKernel>(fn);
+    if constexpr (BN >= 128)
+      return reinterpret_cast<LpKernel>(&gemm_lp_dma16_kernel<T, OutT, BM, BN, false>);
+    else
+      return reinterpret_cast<LpKernel>(&gemm_lp_split_kernel<T, OutT, 4, 4, 4, 1>);
   }
 };
 
@@ -102,12 +175,11 @@ int lp_tile_index(const mcke_gemm_tile* t) {
 
 template <typename T, typename OutT>
 struct LpTable {
-  static int launch(int ti, const void* a, const void* b, void* c, int m, int n, int k,
-                    float alpha, float beta, bool vec, hipStream_t s) {
+  static int launch(int ti, const LpArgs& x, bool vec) {
     switch (ti) {
-      case 0: return LpTile<T, OutT, 256, 256>::launch(a, b, c, m, n, k, alpha, beta, vec, s);
-      case 1: return LpTile<T, OutT, 128, 128>::launch(a, b, c, m, n, k, alpha, beta, vec, s);
-      default: return LpTile<T, OutT, 64, 64>::launch(a, b, c, m, n, k, alpha, beta, vec, s);
+      case 0: return LpTile<T, OutT, 256, 256>::launch(x, vec);
+      case 1: return LpTile<T, OutT, 128, 128>::launch(x, vec);
+      default: return LpTile<T, OutT, 64, 64>::launch(x, vec);
     }
   }
   static LpKernel kernel(int ti) {
@@ -171,14 +243,14 @@ int mcke_launch_gemm_lp(const void* a, const void* b, void* c, int ab_dtype, int
   // the C vector stores need C 16-byte aligned as well.
   const bool vec = (k % 8 == 0) && (n % 8 == 0) && aligned(a, 16) && aligned(b, 16) &&
                    aligned(c, 16);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int mi = static_cast<int>(m), ni = static_cast<int>(n), ki = static_cast<int>(k);
+  const LpArgs x{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), c,
+                 static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), alpha, beta,
+                 static_cast<hipStream_t>(stream)};
   switch (combo) {
-    case 0: return LpTable<__bf16, float>::launch(ti, a, b, c, mi, ni, ki, alpha, beta, vec, s);
-    case 1: return LpTable<__bf16, __bf16>::launch(ti, a, b, c, mi, ni, ki, alpha, beta, vec, s);
-    case 2: return LpTable<_Float16, float>::launch(ti, a, b, c, mi, ni, ki, alpha, beta, vec, s);
-    default:
-      return LpTable<_Float16, _Float16>::launch(ti, a, b, c, mi, ni, ki, alpha, beta, vec, s);
+    case 0: return LpTable<__bf16, float>::launch(ti, x, vec);
+    case 1: return LpTable<__bf16, __bf16>::launch(ti, x, vec);
+    case 2: return LpTable<_Float16, float>::launch(ti, x, vec);
+    default: return LpTable<_Float16, _Float16>::launch(ti, x, vec);
   }
 }
 
@@ -211,13 +283,13 @@ int mcke_gemm_lp_kernel_attrs(int ab_dtype, int c_dtype, const mcke_gemm_tile* t
 int mcke_gemm_lp_default_tile(int64_t m, int64_t n, int64_t k, mcke_gemm_tile* out) {
   if (!out) return invalid("gemm_lp_default_tile: null out");
   (void)k;
-  // The largest tile that still gives every CU of a 256-CU part a workgroup:
-  // measured on MI355X, 256 x 256 wins at 4096^3 (256 tiles) and 128 x 128 at
-  // 2048^3 (256 tiles), each over the next smaller tile with more rounds.
-  const int64_t want = 256;
+  // The largest tile that still fills most of a 256-CU part.  Measured on MI355X: 256 x 256
+  // wins at 4096^3 (256 tiles) and at 3072 x 4096 x 1024 (192 tiles, bf16: 32.1 us against
+  // 33.6), 128 x 128 at 2048^3 (256 tiles: 23.2 us against 37.2 for 64 x 64) and down to
+  // 1628 x 800 (91 tiles), 64 x 64 at 1024^3 (64 tiles of 128: 12.4 us against 8.8).
   auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
-  if (tiles(256) >= want) *out = mcke_gemm_tile{256, 256, kLpBK, 16, 16};
-  else if (tiles(128) >= want) *out = mcke_gemm_tile{128, 128, kLpBK, 8, 8};
+  if (tiles(256) >= 192) *out = mcke_gemm_tile{256, 256, kLpBK, 16, 16};
+  else if (tiles(128) >= 80) *out = mcke_gemm_tile{128, 128, kLpBK, 8, 8};
   else *out = mcke_gemm_tile{64, 64, kLpBK, 4, 4};
   return ok();
 }

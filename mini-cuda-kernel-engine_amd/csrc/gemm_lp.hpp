@@ -1,8 +1,10 @@
 // gemm_lp.hpp -- 16-bit-input GEMM on the CDNA4 matrix cores, fp32 accumulation.
-// Three kernels: gemm_lp_kernel (any shape, register-staged, 32x32x16 MFMAs, the
-// layout described first below), gemm_lp_dma_kernel (whole tiles, direct-to-LDS,
-// 32x32x16, K % 64 == 32) and gemm_lp_dma16_kernel (whole tiles, direct-to-LDS,
-// 16x16x32, K % 64 == 0), each described where it is defined.
+// Kernels: gemm_lp_kernel (any shape, register-staged, 32x32x16 MFMAs, the layout
+// described first below; products narrower than 32 columns take it),
+// gemm_lp_dma_kernel (direct-to-LDS, 32x32x16; whole 128 x 128 tiles with K % 64 == 32),
+// gemm_lp_dma16_kernel (direct-to-LDS, 16x16x32; whole tiles with K % 64 == 0, and an
+// EDGE form for other even shapes), each described where it is defined, and
+// gemm_lp_split_kernel (gemm_lp_split.hpp; small tiles, any alignment).
 //
 // C[M,N] = alpha * A[M,K] B[K,N] + beta * C, row-major; A and B in bf16 or fp16,
 // C in fp32 or in the input type (rounded to nearest even on the store).
@@ -52,6 +54,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+// 16 bytes at any 4-byte address.
+typedef unsigned u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kLpBK = 64;            // K depth of one LDS stage (elements)
 constexpr int kLpRowBytes = 128;     // one LDS row: 64 16-bit values
@@ -364,56 +368,18 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Whole-tile kernel (M % BM == N % BN == K % 32 == 0, 16-byte aligned operands):
-// both operands go straight from global memory into LDS (global_load_lds_dwordx4:
-// one instruction writes its 64 lanes' 16 bytes to 1 KB of contiguous LDS, lane j
-// at byte 16 j), STAGES deep, and B is read back transposed by the LDS
-// (ds_read_b64_tr_b16), so no operand passes through VGPRs or ds_writes.
+// Fragment reads are issued as inline asm and waited on explicitly: the
+// compiler cannot tell that a read of stage ks is disjoint from the DMA still
+// landing in other stages, and would otherwise drain every outstanding load
+// (vmcnt(0)) in front of it.  Each use is behind a wait that re-defines the fragment
+// registers (touch_a, touch_b), so no MFMA that uses them can be scheduled above it.
 //
 // ds_read_b64_tr_b16, per 16-lane group: lane r supplies the address of four
 // consecutive 16-bit values R[r][0..3]; lane 4a + b receives
 // { R[a][b], R[4+a][b], R[8+a][b], R[12+a][b] }.  With lane 4j + a pointing at
 // B[k0 + j][n0 + 4a .. n0 + 4a + 3], lane 4a + b receives column n0 + 4a + b at
 // rows k0 .. k0 + 3: a k-contiguous MFMA B fragment, four values per read, two
-// reads per MFMA.  The 16 lanes of a group are the 16 consecutive columns
-// n0 .. n0 + 15, so here B fragments use the plain column order (lane c of an
-// n-tile is column c).
-//
-// Epilogue layout.  For fp32 C, A is the MFMA's first operand: lane c of a tile
-// holds one column, and the 32 lanes of a half-wave store 128 contiguous bytes of
-// a row per instruction (whole cache lines).  For 16-bit C the operands are
-// swapped, so each MFMA accumulates a transposed 32 x 32 tile in which a lane
-// holds runs of four adjacent columns (one 8-byte store each) -- fewer, wider
-// stores than 2-byte ones, which measure faster there.
-//
-// K is staged 32 deep: sub-step s (0, 1) of a stage covers k = 16 s .. 16 s + 15,
-// lane half h the eight k = 16 s + 8 h + e (e = 0..7) -- one 16-byte chunk of an
-// A row, two transposed reads (e = 4 t + j, t = 0, 1) of B.
-//
-// LDS layouts (per stage; XOR swizzles keep every access conflict-free):
-//   A: BM rows of 64 bytes (4 chunks); chunk q of row r sits at position
-//      q ^ ((r / 4) % 4).  A fragment read covers 32 consecutive rows at one
-//      chunk; any 16 of them hit 16 distinct 16-byte bank groups.
-//   B: 32 rows (k) of BN * 2 bytes, n contiguous; 16-byte chunk c of row k sits
-//      at position c ^ (4 (k % 4)).  A transposed read touches rows
-//      k0 .. k0 + 3 (k0 % 4 == 0) and, per lane half, 32 consecutive columns
-//      (4 chunks): the swizzle puts the four rows' chunk quads on distinct
-//      64-byte bank groups.
-// The DMA source of each lane is chosen so that it lands on these positions.
-//
-// Pipeline: the barrier that publishes stage ks + 1 sits between the two
-// sub-steps of stage ks, so the first fragment reads of stage ks + 1 and the
-// DMA of stage ks + STAGES - 1 are issued under the MFMAs of stage ks's second
-// sub-step, and no fragment read is exposed at a barrier.
-// ---------------------------------------------------------------------------
-// Fragment reads are issued as inline asm and waited on explicitly: the
-// compiler cannot tell that a read of stage ks is disjoint from the DMA still
-// landing in other stages, and would otherwise drain every outstanding load
-// (vmcnt(0)) in front of it.  Nothing else in the kernel reads LDS, so the
-// compiler tracks no LDS read of its own, and lds_wait() is the only wait the
-// fragments need: it waits for every read issued so far and re-defines the
-// fragment registers after the wait, so no MFMA that uses them can be scheduled
-// above it.
+// reads per MFMA.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   // A C-style cast is the address-space cast from the generic pointer.
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
@@ -545,20 +511,15 @@ __device__ __forceinline__ void lp_dma_slot(f32x16 (&acc)[BM / 64][BN / 64],
 }
 
 // ---------------------------------------------------------------------------
-// Whole-tile kernel (M % BM == N % BN == K % 32 == 0, 16-byte aligned operands):
-// both operands go straight from global memory into LDS (global_load_lds_dwordx4:
-// one instruction writes its 64 lanes' 16 bytes to 1 KB of contiguous LDS, lane j
-// at byte 16 j), STAGES deep, and B is read back transposed by the LDS
-// (ds_read_b64_tr_b16), so no operand passes through VGPRs or ds_writes.
+// Whole-tile kernel, 32x32x16 MFMAs, both operands by direct-to-LDS loads, STAGES deep
+// (M % BM == N % BN == K % 32 == 0, 16-byte aligned operands), B read back transposed.
 //
-// ds_read_b64_tr_b16, per 16-lane group: lane r supplies the address of four
-// consecutive 16-bit values R[r][0..3]; lane 4a + b receives
-// { R[a][b], R[4+a][b], R[8+a][b], R[12+a][b] }.  With lane 4j + a pointing at
-// B[k0 + j][n0 + 4a .. n0 + 4a + 3], lane 4a + b receives column n0 + 4a + b at
-// rows k0 .. k0 + 3: a k-contiguous MFMA B fragment, four values per read, two
-// reads per MFMA.  The 16 lanes of a group are the 16 consecutive columns
-// n0 .. n0 + 15, so here B fragments use the plain column order (lane c of an
-// n-tile is column c).
+// For 128 x 128 tiles with K % 64 == 32 only: A's rows are then not whole 128-byte lines
+// apart, and this kernel's 64-byte pieces of them stay inside a line where the 64-deep A
+// buffers of the 16x16x32 kernel straddle two (2048 x 2048 x 2080: 22.8 against 24.4 us
+// for its EDGE form; at 256 x 256, 4096 x 4096 x 4128, the EDGE form leads, 109 against
+// 121 us).  The 16 lanes of a transposed read's group are 16 consecutive columns, so here
+// B fragments use the plain column order (lane c of an n-tile is column c).
 //
 // K is staged 32 deep: sub-step s (0, 1) of a stage covers k = 16 s .. 16 s + 15,
 // lane half h the eight k = 16 s + 8 h + e (e = 0..7) -- one 16-byte chunk of an
@@ -1040,7 +1001,15 @@ __device__ __forceinline__ float acc_get(float a) {
   return v;
 }
 
-template <typename T, typename OutT, int BM, int BN>
+// EDGE: any M, any even N >= BN, any even K >= 64, operands at 4-byte alignment (all that a
+// direct-to-LDS load asks of its source), with the whole-tile loop unchanged:
+//   * rows past M read row M - 1 again and are not stored;
+//   * the last tile column starts at N - BN, so that no load leaves a row of B; the
+//     columns that the tile before it owns are computed again and not stored;
+//   * the K % 64 remainder is the first pair of steps, not the last: its columns are
+//     loaded through registers with bounds checks, zero past them in both operands, and
+//     the whole pairs follow.
+template <typename T, typename OutT, int BM, int BN, bool EDGE = false>
 __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, OutT* __restrict__ C,
     int M, int N, int K, float alpha, float beta, int tiles_m, int tiles_n) {
@@ -1055,7 +1024,9 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
 
   int tm, tn;
   mfma_tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * BM, n_first = tn * BN;
+  const int n0 = EDGE && n_first > N - BN ? N - BN : n_first;
+  const int rem = EDGE ? K % 64 : 0;
 
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
@@ -1069,17 +1040,24 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
   //   + 7 of an A buffer; lane l the chunk at position l % 8 of row l / 8 there,
   //   which holds chunk (l % 8) ^ (row % 8).  row >= 8 q and K >= 64 keep the
   //   difference non-negative.
-  //   B: as gemm_lp_dma_kernel with this kernel's B swizzle; row >=
+  //   B: instruction ii of wave w fills rows kBRowsPerChunk (NB w + ii) on, lane l the chunk
+  //   at position l % kBChunksPerRow of its row, by B's swizzle; row >=
   //   kBRowsPerChunk ii with N >= BN keeps it non-negative.
-  const char* a_base = reinterpret_cast<const char*>(A + static_cast<int64_t>(m0) * K);
-  const char* b_base = reinterpret_cast<const char*>(B + n0);
+  //   EDGE: rows are clamped, so A's offsets are kept non-negative by 3 KB that the base
+  //   gives back; with a remainder, pair p > 0 holds K columns from 64 p - pad on.
+  constexpr uint32_t kBaseA = EDGE ? 3072u : 0u;
+  const int pad = rem ? 64 - rem : 0;
+  const char* a_base = reinterpret_cast<const char*>(A) +
+                       (static_cast<int64_t>(m0) * K - pad) * 2 - static_cast<int64_t>(kBaseA);
+  const char* b_base = reinterpret_cast<const char*>(B) + (n0 - static_cast<int64_t>(pad) * N) * 2;
   const int64_t b_step = static_cast<int64_t>(BK) * N * 2;        // bytes per step
   uint32_t a_src[2 * NA], b_src[S::NB];
 #pragma unroll
   for (int q = 0; q < 2 * NA; ++q) {
-    const int row = 8 * (wave * 2 * NA + q) + lane / 8;
-    const int cg = (lane % 8) ^ (row % 8);
-    a_src[q] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) * 2u + 16u * cg -
+    const int row_t = 8 * (wave * 2 * NA + q) + lane / 8;
+    const int cg = (lane % 8) ^ (row_t % 8);
+    const int row = EDGE && row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
+    a_src[q] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) * 2u + 16u * cg + kBaseA -
                1024u * (q % NA);
   }
 #pragma unroll
@@ -1118,7 +1096,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
 
   const uint32_t lds0 = lds_addr(smem);
   const uint32_t ldsb = lds0 + S::kBBase;
-  const int ksteps = K / BK;                    // even
+  const int ksteps = EDGE ? 2 * ((K + 63) / 64) : K / BK;   // even
   const int last_pair = ksteps / 2 - 1;
   u32x4 av[2][MT];
   u32x2 bv[2][NT][2];
@@ -1145,13 +1123,62 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
     for (int ks = -S::kDepth - 1; ks < 0; ++ks) {
       Lp16Step sp;
       dma_plan(ks, sp);
-      [&]<int... II>(std::integer_sequence<int, II...>) {
-        (S::template dma_a<II>(a_base, a_src, sp.a_pair, sp.a_half, sp.abuf_dma, wave_u), ...);
-      }(std::make_integer_sequence<int, NA>{});
-      if (ks >= -S::kDepth) {
+      // With a remainder, A pair 0 and B steps 0 and 1 are in place.
+      const bool have_a = EDGE && rem && ks < -S::kDepth + 1, have_b = EDGE && rem && ks < -1;
+      if (!have_a) {
+        [&]<int... II>(std::integer_sequence<int, II...>) {
+          (S::template dma_a<II>(a_base, a_src, sp.a_pair, sp.a_half, sp.abuf_dma, wave_u), ...);
+        }(std::make_integer_sequence<int, NA>{});
+      }
+      if (ks >= -S::kDepth && !have_b) {
         [&]<int... II>(std::integer_sequence<int, II...>) {
           (S::template dma_b<II>(b_base, b_step, b_src, sp.b_kstep, sp.bbuf_dma, wave_u), ...);
         }(std::make_integer_sequence<int, S::NB>{});
+      }
+    }
+    if constexpr (EDGE) {
+      if (rem) {
+        // A pair 0 and B steps 0 and 1: the remainder's columns, zero past them.  All
+        // loads go out at once, behind the prologue's DMA; past the remainder they repeat
+        // an address inside it.
+        constexpr int IA = BM * 8 / kMfmaThreads, IB = 64 * BN / 8 / kMfmaThreads;
+        u32x4 va[IA], vb[IB];
+#pragma unroll
+        for (int i = 0; i < IA; ++i) {
+          const int li = i * kMfmaThreads + threadIdx.x;
+          const int row_t = li / 8, k = 8 * ((li % 8) ^ (row_t % 8));
+          const int row = row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
+          const uint16_t* src = A + static_cast<int64_t>(m0 + row) * K;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {     // rem is even
+            const int ke = k + 2 * e < rem ? k + 2 * e : rem - 2;
+            va[i][e] = *reinterpret_cast<const uint32_t*>(src + ke);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+          const int li = i * kMfmaThreads + threadIdx.x;
+          const int kr = li / (BN / 8), cg = (li % (BN / 8)) ^ S::bswz(kr % 32);
+          vb[i] = *reinterpret_cast<const u32x4_a4*>(
+              B + static_cast<int64_t>(kr < rem ? kr : rem - 1) * N + n0 + 8 * cg);
+        }
+#pragma unroll
+        for (int i = 0; i < IA; ++i) {
+          const int li = i * kMfmaThreads + threadIdx.x;
+          const int k = 8 * ((li % 8) ^ ((li / 8) % 8));
+          u32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = k + 2 * e < rem ? va[i][e] : 0u;
+          *reinterpret_cast<u32x4*>(smem + 16 * li) = v;
+        }
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+          const int li = i * kMfmaThreads + threadIdx.x;
+          *reinterpret_cast<u32x4*>(smem + S::kBBase + 16 * li) =
+              li / (BN / 8) < rem ? vb[i] : u32x4{0u, 0u, 0u, 0u};
+        }
+        // The barrier that publishes them is a bare one.
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
     }
     // A pair 0 and B step 0 have landed once the D - 1 younger steps' loads at
@@ -1214,6 +1241,27 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
   asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");
 
   using O = LpOut<OutT>;
+  if constexpr (EDGE && !TRANS) {
+    // As below, without the rows past M and the columns before n_first.
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm * WM + 16 * i + 4 * g + r;
+        if (row >= M) continue;
+        const int col = n0 + wn * WN + r16;
+        OutT* crow = C + static_cast<int64_t>(row) * N + col;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          float v = alpha * acc[i][j][r];
+          if (col + 16 * j < n_first) continue;
+          if (beta != 0.0f) v += beta * O::to_f32(crow[16 * j]);
+          crow[16 * j] = O::from_f32(v);
+        }
+      }
+    }
+    return;
+  }
   if constexpr (!TRANS) {
     // Lane (g, r16) of block (i, j), register r: row wm*WM + 16 i + 4 g + r,
     // column wn*WN + 16 j + r16.  A 16-lane group stores 64 contiguous bytes of a
@@ -1239,8 +1287,9 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
   // adjacent columns.
   struct alignas(4 * sizeof(OutT)) Quad { OutT v[4]; };
   if (beta == 0.0f) {
-    // Staged through the (now idle) stage buffers so that the global stores are
-    // whole rows, as in gemm_lp_dma_kernel.  Chunk q of tile row r sits at
+    // Staged through the (now idle) stage buffers, so the global stores are whole rows:
+    // written straight from the registers, the quads reach each 64-byte row segment in
+    // pieces, and the launch ends with a write burst of partial lines.  Chunk q of tile row r sits at
     // q ^ (r % kChunks): the 16 rows of a half-wave's quads land on 16 distinct
     // chunk positions.
     constexpr int kRowBytes = BN * 2;
@@ -1272,22 +1321,43 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
     for (int r0 = 0; r0 < BM; r0 += kRowsPerPass) {
       const int rt = r0 + threadIdx.x / kChunks;
       const u32x4 v = *reinterpret_cast<const u32x4*>(smem + rt * kRowBytes + ((q ^ (rt % kChunks)) * 16));
-      *reinterpret_cast<u32x4*>(C + static_cast<int64_t>(m0 + rt) * N + n0 + 8 * q) = v;
+      OutT* p = C + static_cast<int64_t>(m0 + rt) * N + n0 + 8 * q;
+      if constexpr (!EDGE) {
+        *reinterpret_cast<u32x4*>(p) = v;
+      } else if (m0 + rt < M) {
+        // N, n0 and n_first are even: columns go in pairs, at 4-byte alignment.
+        if (n0 + 8 * q >= n_first) {
+          *reinterpret_cast<u32x4_a4*>(p) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n0 + 8 * q + 2 * e >= n_first) reinterpret_cast<unsigned*>(p)[e] = v[e];
+        }
+      }
     }
     return;
   }
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
-    OutT* crow = C + static_cast<int64_t>(m0 + wm * WM + 16 * i + r16) * N + n0 + wn * WN + 4 * g;
+    const int row = m0 + wm * WM + 16 * i + r16, col = n0 + wn * WN + 4 * g;
+    if (EDGE && row >= M) continue;
+    OutT* crow = C + static_cast<int64_t>(row) * N + col;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       Quad* dst = reinterpret_cast<Quad*>(crow + 16 * j);
-      const Quad old = *dst;
-      Quad o;
+      Quad old, o;
+      if constexpr (EDGE) __builtin_memcpy(&old, crow + 16 * j, sizeof(old));
+      else old = *dst;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         o.v[e] = O::from_f32(alpha * acc_get(acc[i][j][e]) + beta * O::to_f32(old.v[e]));
-      *dst = o;
+      if constexpr (!EDGE) {
+        *dst = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e += 2)
+          if (col + 16 * j + e >= n_first) __builtin_memcpy(crow + 16 * j + e, &o.v[e], 4);
+      }
     }
   }
 }

@@ -1,0 +1,274 @@
+// gemm_lp_split.hpp -- 16-bit-input GEMM whose waves split K: C = alpha A B + beta C,
+// row-major, bf16 or fp16 in, fp32 accumulation, fp32 or 16-bit C; any M, any N >= the
+// tile's width, any K, any element alignment.
+//
+// For tiles up to 64 x 64 and for shapes the direct-to-LDS kernels do not take.  With a
+// tile this small a 2 x 2 wave grid reads each operand from LDS twice (256 bytes per
+// cycle at 64 x 64 for 16x16x32 MFMAs, twice what LDS delivers) and meets at a barrier
+// for a few MFMAs' worth of work.  Here
+//   * every wave computes the whole 16 MT x 16 NW tile over its own K chunks (32 H deep,
+//     dealt to the WV waves in turn), so a fragment is read from LDS once, and the loop
+//     has no barrier: a wave loads a chunk into registers, writes it to an LDS slot of its
+//     own while the next chunk's loads are in flight, and reads the fragments back;
+//   * loads are 16 bytes per lane at 2-byte alignment, so odd widths and unaligned
+//     operands take the same path (the register-staged kernel loads them 2 bytes at a
+//     time);
+//   * B is transposed by the LDS (ds_read_b64_tr_b16) on the way back;
+//   * the waves' sums are folded through LDS in a fixed order at the end.
+//
+// Measured on MI355X, fp16 to fp32, four sets of operands in turn (us; the
+// register-staged kernel, 64 x 64 tile, then this):
+//   16 x 4096 x 4096  46.6  11.8 (16 x 32, 8 waves)   1024^3           14.9   8.4 (64 x 64)
+//   64 x 4096 x 4096  47.3  17.9 (64 x 32, 8 waves)   317 x 304 x 960  13.4   6.1 (64 x 32)
+//   9 x 5184 x 1523   58.7   8.2 (16 x 64, 8 waves)   1628 x 800 x 1109  77.5  20.4 (64 x 64)
+//   36 x 7379 x 8064   409  42.3 (64 x 32)            4032 x 843 x 2744   254  70.7 (64 x 64)
+// Direct-to-LDS loads in the same scheme are within 6% either way (16 x 4096 x 4096 12.4,
+// 1024^3 7.9) and need 4-byte alignment.
+//
+// LDS slot of a wave, per chunk: H KB per 16 rows of A, rows of 64 H bytes with 16-byte
+// quad q of row r at q ^ aswz(r); per 32 k, NW KB of B: k = 8 g + 4 t + j sits at
+// position s = 16 t + 4 g + j (a transposed read takes one t), 32-byte column block b of
+// a position at b ^ bswz(s).  Both put what a half-wave reads on distinct banks.
+#pragma once
+
+#include "gemm_lp.hpp"
+
+namespace mcke_amd {
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// 16 bytes at any 2-byte address.
+typedef unsigned u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+
+template <int MT, int NW, int WV, int H>
+struct LpSplitShape {
+  static constexpr int TM = 16 * MT, TN = 16 * NW;
+  static constexpr int KC = 32 * H;                       // K per chunk
+  static constexpr int NA = MT * H, NB = NW * H;          // 1 KB loads per chunk
+  static constexpr int L = NA + NB;
+  static constexpr int kSlot = L * 1024;
+  static constexpr int kThreads = WV * 64;
+  static constexpr int kSlots = WV * kSlot;
+  static constexpr int kOut = TM * TN;                    // values of one wave's sums
+  // How many waves' sums fit beside each other: a power of two, all of them if that
+  // takes no more LDS than the slots.
+  static constexpr int kFold = kOut * 4 * WV <= kSlots ? WV : WV / 2;
+  static constexpr int kLds = kSlots > kFold * kOut * 4 ? kSlots : kFold * kOut * 4;
+  static_assert(kLds <= 64 * 1024, "two workgroups or more per CU");
+  static constexpr int kARow = 64 * H, kBRow = 32 * NW;
+  static __host__ __device__ constexpr int aswz(int r) { return H == 2 ? (r >> 1) & 7 : (r >> 2) & 3; }
+  static __host__ __device__ constexpr int bswz(int s) {
+    return NW == 1 ? 0 : NW == 2 ? (s >> 2) & 1 : (s >> 1) & 3;
+  }
+};
+
+template <typename T, typename OutT, int MT, int NW, int WV, int H>
+__global__ __launch_bounds__(WV * 64) void gemm_lp_split_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, OutT* __restrict__ C, int M,
+    int N, int K, float alpha, float beta, int tiles_m, int tiles_n) {
+  using S = LpSplitShape<MT, NW, WV, H>;
+  constexpr int L = S::L;
+  __shared__ __attribute__((aligned(1024))) char smem[S::kLds];
+
+  int tm, tn;
+  mfma_tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * S::TM, n_first = tn * S::TN;
+  const int n0 = n_first > N - S::TN ? N - S::TN : n_first;
+
+  const int lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int g = lane / 16, c = lane % 16;
+
+  // Source byte offsets of this lane's 16 bytes in each 1 KB load of a chunk (the launcher
+  // keeps them in 32 bits).  Rows past M repeat row M - 1 and are not stored; the last tile
+  // column starts at N - TN and stores only the columns of its own.
+  uint32_t a_src[S::NA], b_src[S::NB];
+#pragma unroll
+  for (int i = 0; i < S::NA; ++i) {
+    const int at = (i % H) * 1024 + 16 * lane;
+    const int r = at / S::kARow, row_t = 16 * (i / H) + r;
+    const int row = row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
+    const int q = ((at % S::kARow) / 16) ^ S::aswz(r);
+    a_src[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) * 2u + 16u * q;
+  }
+#pragma unroll
+  for (int u = 0; u < S::NB; ++u) {
+    const int at = (u % NW) * 1024 + 16 * lane;
+    const int s = at / S::kBRow;
+    const int b = ((at % S::kBRow) / 32) ^ S::bswz(s);
+    const int k = 32 * (u / NW) + 8 * ((s / 4) % 4) + 4 * (s / 16) + s % 4;
+    b_src[u] = (static_cast<uint32_t>(k) * static_cast<uint32_t>(N) + 16u * b) * 2u +
+               static_cast<uint32_t>(at % 32);
+  }
+  const char* a_base = reinterpret_cast<const char*>(A + static_cast<int64_t>(m0) * K);
+  const char* b_base = reinterpret_cast<const char*>(B + n0);
+  char* slot = smem + wave * S::kSlot;
+
+  // Fragment addresses within a slot.
+  uint32_t a_off[H], b_off[NW];
+#pragma unroll
+  for (int h = 0; h < H; ++h) a_off[h] = c * S::kARow + 16 * ((4 * h + g) ^ S::aswz(c));
+#pragma unroll
+  for (int b = 0; b < NW; ++b) {
+    const int s = g * 4 + c / 4;                        // read t adds 16 positions
+    b_off[b] = S::NA * 1024 + s * S::kBRow + 32 * (b ^ S::bswz(s)) + 8 * (c % 4);
+  }
+
+  f32x4 acc[MT][NW];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int b = 0; b < NW; ++b) acc[i][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int chunks = K / S::KC;
+  const int n_it = chunks > wave ? (chunks - wave + WV - 1) / WV : 0;
+  auto compute = [&]() {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      u32x4 av[MT];
+      u32x2 bv[NW][2];
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        av[m] = *reinterpret_cast<const u32x4*>(slot + m * (H * 1024) + a_off[h]);
+#pragma unroll
+      for (int b = 0; b < NW; ++b)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          bv[b][t] = __builtin_bit_cast(
+              u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                         (__attribute__((address_space(3))) s16x4*)(
+                             slot + h * (NW * 1024) + t * (16 * S::kBRow) + b_off[b])));
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int bb = 0; bb < NW; ++bb) {
+          const int b = mfma_snake_col(m, bb, NW);
+          acc[m][b] = LpMfma16<T>::run(
+              av[m], u32x4{bv[b][0][0], bv[b][0][1], bv[b][1][0], bv[b][1][1]}, acc[m][b]);
+        }
+    }
+  };
+
+  if (n_it > 0) {
+    u32x4 v[L];
+    auto load = [&](int it) {
+      const int64_t k0 = static_cast<int64_t>(S::KC) * (wave + WV * it);
+      const char* ap = a_base + k0 * 2;
+      const char* bp = b_base + k0 * N * 2;
+#pragma unroll
+      for (int i = 0; i < S::NA; ++i) v[i] = *reinterpret_cast<const u32x4_a2*>(ap + a_src[i]);
+#pragma unroll
+      for (int u = 0; u < S::NB; ++u)
+        v[S::NA + u] = *reinterpret_cast<const u32x4_a2*>(bp + b_src[u]);
+    };
+    load(0);
+    for (int it = 0; it < n_it; ++it) {
+      // The slot's last reads have been waited for by the MFMAs that used them.
+#pragma unroll
+      for (int i = 0; i < L; ++i) *reinterpret_cast<u32x4*>(slot + i * 1024 + 16 * lane) = v[i];
+      load(it + 1 < n_it ? it + 1 : it);
+      // Lanes read what other lanes of the wave wrote.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      compute();
+    }
+  }
+
+  const int rem = K % S::KC;
+  if (rem && wave == chunks % WV) {
+    const int64_t k0 = static_cast<int64_t>(chunks) * S::KC;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      u32x4 av[MT], bv[NW];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const int row_t = 16 * m + c;
+        const int row = row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
+        const uint16_t* p = A + static_cast<int64_t>(m0 + row) * K + k0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = 32 * h + 8 * g + 2 * e;
+          const unsigned lo = k < rem ? p[k] : 0u, hi = k + 1 < rem ? p[k + 1] : 0u;
+          av[m][e] = lo | (hi << 16);
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < NW; ++b) {
+        const uint16_t* p = B + k0 * N + n0 + 16 * b + c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = 32 * h + 8 * g + 2 * e;
+          const unsigned lo = k < rem ? p[static_cast<int64_t>(k) * N] : 0u;
+          const unsigned hi = k + 1 < rem ? p[static_cast<int64_t>(k + 1) * N] : 0u;
+          bv[b][e] = lo | (hi << 16);
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int b = 0; b < NW; ++b) acc[m][b] = LpMfma16<T>::run(av[m], bv[b], acc[m][b]);
+    }
+  }
+
+  // The waves' sums.  While there are more than fit, the upper half hands its own to the
+  // lower half; then kFold of them lie side by side and every lane adds them up for the
+  // outputs it stores.  Lane (g, c), register r of block (m, b): row 16 m + 4 g + r,
+  // column 16 b + c.
+  float* sums = reinterpret_cast<float*>(smem);
+  auto at = [&](int w, int m, int b, int r) {
+    return w * S::kOut + ((m * NW + b) * 4 + r) * 64 + lane;
+  };
+  auto put = [&](int w) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int b = 0; b < NW; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sums[at(w, m, b, r)] = acc[m][b][r];
+  };
+  __syncthreads();
+  if constexpr (S::kFold < WV) {
+    static_assert(2 * S::kFold == WV, "one hand-over");
+    if (wave >= S::kFold) put(wave - S::kFold);
+    __syncthreads();
+    if (wave < S::kFold) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int b = 0; b < NW; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[m][b][r] += sums[at(wave, m, b, r)];
+    }
+    // Each wave overwrites only the sums that it has just read.
+  }
+  if (wave < S::kFold) put(wave);
+  __syncthreads();
+  using O = LpOut<OutT>;
+  struct Pack { OutT v[4]; };   // four adjacent columns at any address
+  for (int q = threadIdx.x; q < S::kOut / 4; q += S::kThreads) {
+    const int rt = q / (S::TN / 4), cq = q % (S::TN / 4);
+    const int row = m0 + rt, col = n0 + 4 * cq;
+    if (row >= M || col + 3 < n_first) continue;
+    const int o = (((rt / 16) * NW + cq / 4) * 4 + rt % 4) * 64 + 16 * ((rt / 4) % 4) + 4 * (cq % 4);
+    f32x4 s = *reinterpret_cast<const f32x4*>(sums + o);
+#pragma unroll
+    for (int w = 1; w < S::kFold; ++w)
+      s += *reinterpret_cast<const f32x4*>(sums + w * S::kOut + o);
+    OutT* p = C + static_cast<int64_t>(row) * N + col;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      s[j] *= alpha;
+      if (beta != 0.0f && col + j >= n_first) s[j] += beta * O::to_f32(p[j]);
+    }
+    if (col >= n_first) {
+      Pack out;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) out.v[j] = O::from_f32(s[j]);
+      __builtin_memcpy(p, &out, sizeof(out));
+    } else {
+#pragma unroll
+      for (int j = 1; j < 4; ++j)
+        if (col + j >= n_first) p[j] = O::from_f32(s[j]);
+    }
+  }
+}
+
+}  // namespace mcke_amd

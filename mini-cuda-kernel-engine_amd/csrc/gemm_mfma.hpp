@@ -912,37 +912,6 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
   const int ksteps = EDGE ? (K + BK - 1) / BK : K / BK;
-  if constexpr (EDGE) {
-    if (rem) {
-      // Stage 0: the remainder's columns, zero past them, in the stage's layout.
-      constexpr int T = kDmaThreads<BM, BN, KS>;
-#pragma unroll 4
-      for (int li = threadIdx.x; li < BM * 8; li += T) {
-        const int row_t = li / 8, p = li % 8;
-        const int row = row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
-        const int k = 4 * (p ^ (row_t & 7) ^ ((row_t >> 3) & 1));
-        const float* src = A + static_cast<int64_t>(m0 + row) * K + k;
-        f32x4 v{0.0f, 0.0f, 0.0f, 0.0f};
-        if (k + 4 <= rem) {
-          v = ld4(src);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 3; ++e)
-            if (k + e < rem) v[e] = src[e];
-        }
-        *reinterpret_cast<f32x4*>(smem + 4 * li) = v;
-      }
-#pragma unroll 4
-      for (int li = threadIdx.x; li < BK * BN / 4; li += T) {
-        const int kr = li / (BN / 4), c4 = li % (BN / 4);
-        f32x4 v{0.0f, 0.0f, 0.0f, 0.0f};
-        if (kr < rem) v = ld4(B + static_cast<int64_t>(kr) * N + n0 + 4 * c4);
-        *reinterpret_cast<f32x4*>(smem + kAFloats + 4 * li) = v;
-      }
-      // The barrier that publishes stage 0 is a bare one.
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-  }
   // Prologue: stages 0 .. STAGES-2 in flight.  Past the last K step a stage
   // re-fetches the last one into a buffer nobody reads, which keeps the number of
   // loads per stage -- and so the vmcnt arithmetic below -- uniform.
@@ -956,6 +925,49 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
                                    lds0 + st * kStageFloats * 4, kk, wave_u),
          ...);
       }(std::make_integer_sequence<int, L>{});
+    }
+  }
+
+  if constexpr (EDGE) {
+    if (rem) {
+      // Stage 0: the remainder's columns, zero past them, in the stage's layout.  All loads
+      // go out at once, behind the prologue's DMA; past the remainder they repeat an
+      // address inside it.
+      constexpr int T = kDmaThreads<BM, BN, KS>;
+      constexpr int IA = BM * 8 / T, IB = BK * BN / 4 / T;
+      f32x4 va[IA], vb[IB];
+#pragma unroll
+      for (int i = 0; i < IA; ++i) {
+        const int li = i * T + threadIdx.x;
+        const int row_t = li / 8, k = 4 * ((li % 8) ^ (row_t & 7) ^ ((row_t >> 3) & 1));
+        const int row = row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
+        const float* src = A + static_cast<int64_t>(m0 + row) * K;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) va[i][e] = src[k + e < rem ? k + e : rem - 1];
+      }
+#pragma unroll
+      for (int i = 0; i < IB; ++i) {
+        const int li = i * T + threadIdx.x;
+        const int kr = li / (BN / 4), c4 = li % (BN / 4);
+        vb[i] = ld4(B + static_cast<int64_t>(kr < rem ? kr : rem - 1) * N + n0 + 4 * c4);
+      }
+#pragma unroll
+      for (int i = 0; i < IA; ++i) {
+        const int li = i * T + threadIdx.x;
+        const int row_t = li / 8, k = 4 * ((li % 8) ^ (row_t & 7) ^ ((row_t >> 3) & 1));
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = k + e < rem ? va[i][e] : 0.0f;
+        *reinterpret_cast<f32x4*>(smem + 4 * li) = v;
+      }
+#pragma unroll
+      for (int i = 0; i < IB; ++i) {
+        const int li = i * T + threadIdx.x;
+        *reinterpret_cast<f32x4*>(smem + kAFloats + 4 * li) =
+            li / (BN / 4) < rem ? vb[i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+      // The barrier that publishes stage 0 is a bare one.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   }
 

@@ -1,0 +1,108 @@
+"""GPU parity of the 16-bit GEMM at shapes that are not whole tiles: the EDGE form of the
+direct-to-LDS kernel and the split-K kernel, around their tiles, K steps and limits, with
+operands and C at every element offset, C between guard values that must keep their bits.
+
+Bars: quarter-multiple inputs make every sum exact in fp32, so the result is the oracle's
+bit for bit; infinities and NaN reach their own outputs only.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_gemm_lp import BF16, DT_ID, DTS, F16, F32, _quarters
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 16
+
+# EDGE at 128 x 128 takes even N >= 128 and K >= 64 from 80 tiles on, at 256 x 256 from 192
+# tiles on; K % 64 is its first pair of steps (0, 2, 30, 32, 62 left over).
+EDGE_128 = [(1279, 1024, 64), (1151, 1150, 66), (1025, 1154, 94), (10200, 130, 160),
+            (129, 10112, 126)]
+EDGE_256 = [(3073, 4000, 66), (3100, 4098, 128)]
+# Split K: 16 and 32 rows (8 waves), 32 x 64 and 64 x 64 tiles (past 1024 of 32 x 64), odd
+# widths, K around its 32-deep chunks dealt to 4 and 8 waves; N below 32: register-staged.
+SPLIT = [(1, 32, 1), (16, 33, 31), (15, 8191, 33), (17, 100, 257), (32, 63, 256), (33, 63, 96),
+         (33, 64, 32), (65, 131, 65), (200, 136, 264), (127, 1001, 127), (257, 9001, 63),
+         (5, 8193, 70), (3001, 1501, 35), (40, 31, 64), (7, 5, 3)]
+
+
+def _check(m, orc, dt, out, M, N, K, tile, shifts, alpha, beta):
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
+    a16 = orc.to_16(_quarters(rng, (M, K)), dt)
+    b16 = orc.to_16(_quarters(rng, (K, N)), dt)
+    cf = _quarters(rng, (M, N))
+    cd = F32 if out == "f32" else dt
+    ct = np.float32 if cd == F32 else np.uint16
+    c = cf.ravel() if cd == F32 else orc.to_16(cf, dt).ravel()
+    # The oracle's value in float64 (exact: quarter multiples), rounded as C is.
+    want = alpha * (orc.from_16(a16, dt).reshape(M, K).astype(np.float64) @
+                    orc.from_16(b16, dt).reshape(K, N).astype(np.float64)) + beta * cf
+    want = want.astype(np.float32).ravel()
+    want = want if cd == F32 else orc.to_16(want, dt).ravel()
+    nan16 = 0x7FC0 if dt == BF16 else 0x7E00
+    bufs = []
+
+    def up(arr, shift):
+        pad = np.full(GUARD, nan16, np.uint16)
+        buf = m.DeviceBuffer.from_array(np.concatenate([pad, pad[:shift], arr.ravel(), pad]))
+        bufs.append(buf)
+        return buf.ptr + 2 * (GUARD + shift)
+
+    pa, pb = up(a16, shifts[0]), up(b16, shifts[1])
+    at = GUARD + shifts[2]
+    mark = np.full(at + M * N + GUARD, 77, ct)
+    mark[at:at + M * N] = c if beta != 0.0 else (np.nan if cd == F32 else nan16)
+    dc = m.DeviceBuffer.from_array(mark)
+    st = m.launch_gemm_lp(pa, pb, dc.ptr + at * mark.itemsize, dt, cd, M, N, K, alpha, beta, tile)
+    assert st.ok(), str(st)
+    m.device_synchronize()
+    full = dc.download(mark.size, ct)
+    where = f"{M}x{N}x{K} {DT_ID[dt]}->{out} {tile} shifts={shifts} beta={beta}"
+    assert (full[:at] == 77).all() and (full[at + M * N:] == 77).all(), "wrote outside C: " + where
+    got = full[at:at + M * N]
+    bits = np.uint32 if cd == F32 else np.uint16
+    bad = np.nonzero(got.view(bits) != want.view(bits))[0]
+    assert bad.size == 0, f"{where}: {bad.size} wrong, first at {divmod(int(bad[0]), N)}"
+
+
+@pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
+@pytest.mark.parametrize("out", ["f32", "same"])
+@pytest.mark.parametrize("shape", EDGE_128 + EDGE_256, ids=lambda s: "x".join(map(str, s)))
+def test_edge_tiles(gpu, orc, dt, out, shape):
+    tile = gpu.LP_TILES[0] if shape in EDGE_256 else gpu.LP_TILES[1]
+    _check(gpu, orc, dt, out, *shape, tile, (0, 0, 0), 1.0, 0.0)
+    _check(gpu, orc, dt, out, *shape, tile, (2, 4, 2), 0.5, 2.0)
+
+
+@pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
+@pytest.mark.parametrize("out", ["f32", "same"])
+@pytest.mark.parametrize("shape", SPLIT, ids=lambda s: "x".join(map(str, s)))
+def test_split_k(gpu, orc, dt, out, shape):
+    _check(gpu, orc, dt, out, *shape, gpu.LP_TILES[2], (0, 0, 0), 1.0, 0.0)
+    _check(gpu, orc, dt, out, *shape, gpu.LP_TILES[2], (1, 3, 1), 0.5, 2.0)
+
+
+def test_remainders_keep_special_values_apart(gpu, orc):
+    """The K remainder pads both operands with zeros: infinities and NaN in the last columns
+    of A and the last rows of B reach their own outputs only."""
+    for M, N, K, tile in ((1279, 1026, 70, gpu.LP_TILES[1]), (37, 131, 45, gpu.LP_TILES[2])):
+        rng = np.random.default_rng(K)
+        a, b = _quarters(rng, (M, K)), _quarters(rng, (K, N))
+        a[M - 1, 3], a[0, K - 1] = np.nan, np.inf
+        b[K - 1, N - 1] = -np.inf
+        b[K - 1, 0] = 0.25
+        a16, b16 = orc.to_16(a, F16), orc.to_16(b, F16)
+        with np.errstate(invalid="ignore"):
+            want = (np.einsum("mk,kn->mn", a.astype(np.float64), b.astype(np.float64))
+                    .astype(np.float32))
+        da, db = gpu.DeviceBuffer.from_array(a16), gpu.DeviceBuffer.from_array(b16)
+        dc = gpu.DeviceBuffer(M * N * 4)
+        st = gpu.launch_gemm_lp(da, db, dc, F16, F32, M, N, K, 1.0, 0.0, tile)
+        assert st.ok(), str(st)
+        gpu.device_synchronize()
+        got = dc.download(M * N).reshape(M, N)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        assert np.array_equal(got[ok], want[ok])
