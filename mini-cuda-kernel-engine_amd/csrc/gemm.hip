@@ -428,32 +428,46 @@ int launch_rocblas(const float* a, const float* b, float* c, int m, int n, int k
   return ok();
 }
 
-using RowsFn = void (*)(const float*, const float*, float*, int, int, int, float, float, EpiArgs);
+using RowsFn = void (*)(const float*, const float*, float*, int, int, int, float, float, int, int,
+                        EpiArgs);
 
-// The few-rows kernel for a 32 x 32 tile launch, if it is the better one, and its column
-// width: the narrowest of 16, 32 and 64 columns a workgroup whose workgroups are all
-// resident at once.  Wider ones, or more row blocks than two, pay off from K = 1024 on
-// (7 x 6015 x 628: 7.4 against 7.3 us for the tile; 64 x 4096 x 256: 5.0 against 4.4;
-// 32 x 8192 x 1024: 9.4 against 10.4).  Past 64 rows the product is bound by the MFMAs.
-// Per-lane source offsets are 32-bit.
-RowsFn find_rows(int64_t m, int64_t n, int64_t k, bool fused, int* width) {
-  if (m > 64 || n < 16 || k < 1 || 64 * k >= (int64_t{1} << 30)) return nullptr;
+// The few-tiles kernel for a 32 x 32 tile launch, if it is the better one: the smallest of
+// its tiles (16 x 16, 16 x 32, 32 x 32, and 16 x 64 for up to 16 rows) whose workgroups
+// are all resident at once, one per CU.  More than that is slower (300 x 217 x 4072: 266
+// tiles of 16 x 16 27.1 us, 133 of 16 x 32 19.3).  The wider ones need some K to pay for
+// their sums: 16 x 32 ties at 7 x 6015 x 628 (7.4 us against 7.3 for the 32 x 32 tile) and
+// leads at 128 x 1012 x 320 (4.4 against 4.5); 32 x 32 leads from K = 1024 on (512 x 512 x
+// 1024: 7.7 against 8.7; 500 x 500 x 1000: 9.9 against 9.6); 16 x 64 trails at 16 x 16384 x
+// 256 (6.1 against 5.6) and leads at 16 x 16384 x 4096.  Per-lane source offsets are 32-bit.
+struct RowsPick {
+  RowsFn fn = nullptr;
+  int tiles_m = 0, tiles_n = 0;
+};
+
+RowsPick find_rows(int64_t m, int64_t n, int64_t k, bool fused) {
+  RowsPick p;
+  if (64 * k >= (int64_t{1} << 30) || 64 * n >= (int64_t{1} << 30)) return p;
   const int64_t cus = device_cu_count();
-  const int nw = (n + 15) / 16 <= cus ? 1 : (n + 31) / 32 <= cus ? 2 : 4;
-  if ((n + 16 * nw - 1) / (16 * nw) > cus) return nullptr;
-  const int mt = m <= 16 ? 1 : m <= 32 ? 2 : 4;
-  if ((nw > 1 || mt > 2) && k < 1024) return nullptr;
-  *width = 16 * nw;
-#define MCKE_ROWS(MT, NW) \
-  if (mt == MT && nw == NW) \
-    return fused ? &gemm_rows_kernel<MT, NW, true> : &gemm_rows_kernel<MT, NW, false>;
-  MCKE_ROWS(1, 1) MCKE_ROWS(1, 2) MCKE_ROWS(1, 4)
-  MCKE_ROWS(2, 1) MCKE_ROWS(2, 2) MCKE_ROWS(4, 1)
+  auto fits = [&](int mt, int nw, int64_t min_k) {
+    const int64_t tm = (m + 16 * mt - 1) / (16 * mt), tn = (n + 16 * nw - 1) / (16 * nw);
+    p.tiles_m = static_cast<int>(tm);
+    p.tiles_n = static_cast<int>(tn);
+    return n >= 16 * nw && k >= min_k && tm * tn <= cus;
+  };
+#define MCKE_ROWS(MT, NW, MIN_K)                                                              \
+  if (fits(MT, NW, MIN_K)) {                                                                  \
+    p.fn = fused ? &gemm_rows_kernel<MT, NW, true> : &gemm_rows_kernel<MT, NW, false>;        \
+    return p;                                                                                 \
+  }
+  MCKE_ROWS(1, 1, 1)
+  MCKE_ROWS(1, 2, 320)
+  MCKE_ROWS(2, 2, 1024)
+  if (m <= 16) MCKE_ROWS(1, 4, 1024)
 #undef MCKE_ROWS
-  return nullptr;   // more rows at wider columns: the tile
+  return p;
 }
 
-// One kMfmaF32 launch: few rows at the 32 x 32 tile take the few-rows kernel, whole tiles
+// One kMfmaF32 launch: few tiles of 32 x 32 take the few-tiles kernel, whole tiles
 // the direct-to-LDS kernel, and other shapes its EDGE form where a tile's columns fit in a
 // row of B and K holds a stage, else the staged kernel; `fused` picks the instantiations
 // with the bias + activation epilogue, which route shapes exactly as the plain ones do
@@ -463,13 +477,15 @@ int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, con
                 hipStream_t s) {
   // The kernels below load and store floats at 4-byte addresses.
   const bool floats = aligned(a, 4) && aligned(b, 4) && aligned(c, 4) && aligned(epi.bias, 4);
-  int width = 0;
-  const RowsFn rows_fn = sp.tile_m == 32 && floats ? find_rows(m, n, k, fused, &width) : nullptr;
-  if (rows_fn) {
-    rows_fn<<<static_cast<unsigned>((n + width - 1) / width), kRowsThreads, 0, s>>>(
-        a, b, c, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), alpha, beta, epi);
-    MCKE_LAUNCH_CHECK(fused ? "gemm_rows_kernel (bias + activation)" : "gemm_rows_kernel");
-    return ok();
+  if (sp.tile_m == 32 && floats && k > 0) {
+    const RowsPick p = find_rows(m, n, k, fused);
+    if (p.fn) {
+      p.fn<<<static_cast<unsigned>(p.tiles_m * p.tiles_n), kRowsThreads, 0, s>>>(
+          a, b, c, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), alpha, beta,
+          p.tiles_m, p.tiles_n, epi);
+      MCKE_LAUNCH_CHECK(fused ? "gemm_rows_kernel (bias + activation)" : "gemm_rows_kernel");
+      return ok();
+    }
   }
   const int64_t tiles_m = (m + sp.tile_m - 1) / sp.tile_m;
   const int64_t tiles_n = (n + sp.tile_n - 1) / sp.tile_n;

@@ -1,25 +1,28 @@
-// gemm_rows.hpp -- fp32 GEMM with few rows (M <= 16 MT): C = alpha A B + beta C, or the
+// gemm_rows.hpp -- fp32 GEMM for products with few tiles: C = alpha A B + beta C, or the
 // fused bias + activation form, row-major.
 //
-// Such a product is bound by reading B once (4 K N bytes).  The 32 x 32 tile gives a
-// launch one workgroup per 32 columns, meets at a barrier every 32 of K, and spends half
-// or more of its MFMA rows on padding.  Here
-//   * a workgroup owns W = 16 NW columns and all of K, so that 4096 columns are 256
-//     workgroups, and its 8 waves take the 32-deep K chunks in turn;
+// A product of a few rows is bound by reading B once (4 K N bytes), and a small one by how
+// few CUs its tiles reach.  The 32 x 32 tile gives either a workgroup per 32 columns and 32
+// rows, four waves each, that meet at a barrier every 32 of K, and spends half or more of
+// its MFMA rows on padding if there are 16 rows or less.  Here
+//   * a workgroup owns 16 MT rows, W = 16 NW columns and all of K, so that 16 x 4096 is
+//     256 workgroups, and its 8 waves take the 32-deep K chunks in turn;
 //   * each wave streams its chunks into a ring of its own in LDS by direct-to-LDS loads,
 //     with no barrier in the loop (a wave waits for its own loads only);
 //   * v_mfma_f32_16x16x4_f32: 16 rows of A per instruction instead of 32;
 //   * the waves' sums are added in wave order through LDS at the end.
 //
-// Measured with four B matrices in turn (us; the 32 x 32 tile, then this):
-//   16 x 4096 x 4096   28.9  15.6 (NW 1; a plain read of B takes 10.8)
-//   16 x 8192 x 8192   79.5  54.6 (NW 2)      16 x 16384 x 4096  53.6  47.8 (NW 4)
-//   32 x 4096 x 4096   29.7  18.4 (MT 2)      48 x 4096 x 4096   29.0  22.5 (MT 4)
-//   13 x 1105 x 1992   14.8   9.1             4 x 259 x 360       4.7   3.3
+// Measured with four sets of operands in turn (us; the 32 x 32 tile, then this):
+//   16 x 4096 x 4096   28.9  15.6 (MT 1, NW 1; a plain read of B takes 10.8)
+//   16 x 8192 x 8192   79.5  54.6 (1, 2)      16 x 16384 x 4096  53.6  47.8 (1, 4)
+//   32 x 4096 x 4096   29.2  17.1 (1, 2)      64 x 4096 x 4096   29.3  21.7 (2, 2)
+//   4 x 259 x 360       4.7   3.3 (1, 1)      96 x 96 x 8000     47.8  17.5 (1, 1)
+//   300 x 217 x 4072   27.6  19.3 (1, 2)      512 x 512 x 2048   14.7  11.7 (2, 2)
 // Chunks are 32 deep so that A's 128-byte pieces are whole cache lines: every workgroup
-// reads all of A, and with 16-deep chunks (64-byte pieces) the first row took 17.2 us.
-// Rings deeper than two chunks are slower (three: 16.3, four: 16.6): what is in flight is
-// enough, and shallow rings keep neighbours, which share lines of B at NW 1, together.
+// reads all of its rows of A, and with 16-deep chunks (64-byte pieces) the first line took
+// 17.2 us.  Rings deeper than two chunks are slower (three: 16.3, four: 16.6): what is in
+// flight is enough, and shallow rings keep neighbours, which share lines of B at NW 1,
+// together.
 //
 // Fragments.  One 16x16x4 MFMA takes, per lane l (g = l / 16, c = l % 16), A[c][k_g] and
 // B[k_g][c] for the four lane groups' k_g.  MFMA i (0 .. 3) of a chunk's half h uses
@@ -30,9 +33,9 @@
 // h, 64-byte column block b of a position at b ^ x(p).  The four rows of B that an MFMA
 // reads are then neighbours on distinct banks, and so are the quads of A.
 //
-// Any M up to 16 MT (rows past it repeat the last one and are not stored), any N >= W
-// (the last workgroup starts at N - W and stores only the columns of its own), any K (its
-// last K % 32 go through registers), 4-byte alignment.
+// Any M (rows past it repeat the last one and are not stored), any N >= W (the last tile
+// column starts at N - W and stores only the columns of its own), any K (its last K % 32
+// go through registers), 4-byte alignment.
 #pragma once
 
 #include "gemm_mfma.hpp"
@@ -47,7 +50,7 @@ constexpr int kRowsDepth = 2;
 template <int MT, int NW, bool FUSED>
 __global__ __launch_bounds__(kRowsThreads, 1) void gemm_rows_kernel(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N,
-    int K, float alpha, float beta, EpiArgs epi) {
+    int K, float alpha, float beta, int tiles_m, int tiles_n, EpiArgs epi) {
   constexpr int W = 16 * NW;
   constexpr int D = kRowsDepth;
   constexpr int L = 2 * (MT + NW);           // direct-to-LDS instructions per chunk
@@ -57,13 +60,13 @@ __global__ __launch_bounds__(kRowsThreads, 1) void gemm_rows_kernel(
   static_assert(MT * NW <= D * L, "the waves' sums must fit in the rings");
 
   // Neighbouring workgroups share cache lines of B where W is less than a line: each XCD
-  // (workgroup id % 8) takes a contiguous run of columns.
-  const int n_wg = gridDim.x;
-  const int full = n_wg - n_wg % kXcds;
-  const int id = blockIdx.x;
-  const int t = id < full ? (id % kXcds) * (full / kXcds) + id / kXcds : id;
-  const int n_first = t * W;
+  // takes a contiguous run of columns.
+  int tm, tn;
+  mfma_tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * 16 * MT, n_first = tn * W;
   const int n0 = n_first > N - W ? N - W : n_first;
+  const int last = M - 1 - m0;               // rows past it repeat it
+  A += static_cast<int64_t>(m0) * K;
 
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -73,7 +76,7 @@ __global__ __launch_bounds__(kRowsThreads, 1) void gemm_rows_kernel(
   uint32_t a_src[2 * MT], b_src[2 * NW];
 #pragma unroll
   for (int i = 0; i < 2 * MT; ++i) {
-    const int r = 8 * i + lane / 8, row = r < M ? r : M - 1;
+    const int r = 8 * i + lane / 8, row = r < last ? r : last;
     const int quad = (lane % 8) ^ ((r % 16) >> 1);
     a_src[i] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(K) + 4u * quad) * 4u;
   }
@@ -165,7 +168,7 @@ __global__ __launch_bounds__(kRowsThreads, 1) void gemm_rows_kernel(
       float av[MT], bv[NW];
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        const int row = 16 * m + c < M ? 16 * m + c : M - 1;
+        const int row = 16 * m + c < last ? 16 * m + c : last;
         av[m] = in ? A[static_cast<int64_t>(row) * K + k0 + k] : 0.0f;
       }
 #pragma unroll
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(kRowsThreads, 1) void gemm_rows_kernel(
   __syncthreads();
   for (int o = threadIdx.x; o < kOut; o += kRowsThreads) {
     const int blk = o / 256, r = (o / 64) % 4, l = o % 64;
-    const int row = 16 * (blk / NW) + 4 * (l / 16) + r;
+    const int row = m0 + 16 * (blk / NW) + 4 * (l / 16) + r;
     const int col = n0 + 16 * (blk % NW) + l % 16;
     if (row >= M || col < n_first) continue;
     float s = sums[o];

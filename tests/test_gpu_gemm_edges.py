@@ -99,13 +99,14 @@ def test_gemm_remainder_keeps_special_values_apart(gpu, orc, t):
     assert orc.compare(got[fin], want[fin], orc.tol_gemm(K), orc.abs_tol_gemm(K)).ok
 
 
-# (M, N, K) around the few-rows kernel's row blocks (16, 32, 64), column widths (16 up to
-# 4096 columns, 32 and 64 past 4096 and 8192 from K = 1024 on), K chunks (32, dealt to 8
-# waves) and its limits (65 rows, 15 columns: the tile kernels).
+# (M, N, K) around the few-tiles kernel's tiles (16 x 16 while 256 of them hold the product,
+# then 16 x 32 from K = 320 on, 32 x 32 from K = 1024 on, 16 x 64 up to 16 rows), K chunks
+# (32, dealt to 8 waves) and limits (15 columns, more than 256 tiles: the tile kernels).
 ROWS_SHAPES = [(1, 16, 1), (16, 17, 31), (17, 31, 32), (31, 33, 33), (32, 100, 255), (33, 64, 1024),
                (48, 77, 1031), (64, 259, 1056), (15, 4095, 257), (16, 4096, 256), (5, 4097, 1024),
                (16, 4128, 1027), (32, 8192, 1025), (3, 8193, 1055), (16, 16383, 1024),
-               (65, 40, 300), (7, 15, 90)]
+               (65, 40, 300), (7, 15, 90), (255, 255, 70), (300, 217, 321), (193, 771, 1056),
+               (512, 512, 1055), (2000, 33, 333), (257, 256, 64)]
 
 
 @pytest.mark.parametrize("shape", ROWS_SHAPES, ids=lambda s: "x".join(map(str, s)))
