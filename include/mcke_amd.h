@@ -171,7 +171,8 @@ int mcke_launch_row_softmax_f32(const float* x, float* y, int64_t rows, int64_t 
  * C = alpha*A[m,k]B[k,n] + beta*C, row-major.  C is not read when beta == 0.
  * m == 0 or n == 0 is a no-op; k == 0 gives C = beta*C.  a == c or b == c,
  * negative or > INT32_MAX extents, and (variant, tile) pairs that are not
- * compiled are INVALID_ARGUMENT (no fallback tile). */
+ * compiled are INVALID_ARGUMENT (no fallback tile).  kMfmaF32's 32 x 32 and 64 x 64 tiles name
+ * a size class: a launch runs the class's kernel whose tiles fill the GPU best. */
 int mcke_launch_gemm_f32(const float* a, const float* b, float* c, int64_t m, int64_t n,
                          int64_t k, float alpha, float beta, int variant,
                          const mcke_gemm_tile* tile, void* stream);

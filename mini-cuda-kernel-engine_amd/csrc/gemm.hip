@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 #include <utility>
@@ -292,6 +293,55 @@ const MfmaCfg kMfmaCfgs[] = {
 #undef MCKE_MFMA_CFG
 #undef MCKE_MFMA_CFG_DMA
 
+// Direct-to-LDS kernels that a 64 x 64 launch runs where their tiles fill the CUs better
+// (tile_us below): 128 x 64 at 144 against 138 TFLOP/s where there are tiles enough, and
+// 32 x 64 (two wave groups over K) at 128 TFLOP/s where 64 x 64 tiles leave CUs with one
+// against others' two.  Block sizes are all kMfmaThreads.
+struct SubTile {
+  int bm, bn;
+  MfmaFn even, edge, even_f, edge_f;
+};
+#define MCKE_SUB(BM, BN, ST, KS)                                                       \
+  {BM, BN, &gemm_mfma_dma_kernel<BM, BN, ST, KS, false, false>,                        \
+   &gemm_mfma_dma_kernel<BM, BN, ST, KS, false, true>,                                 \
+   &gemm_mfma_dma_kernel<BM, BN, ST, KS, true, false>,                                 \
+   &gemm_mfma_dma_kernel<BM, BN, ST, KS, true, true>}
+const SubTile kSubTiles64[] = {MCKE_SUB(128, 64, 2, 1), MCKE_SUB(32, 64, 4, 2)};
+#undef MCKE_SUB
+static_assert(kDmaThreads<128, 64, 1> == kMfmaThreads && kDmaThreads<32, 64, 2> == kMfmaThreads &&
+                  kDmaThreads<64, 64, 1> == kMfmaThreads,
+              "one block size");
+
+// What a launch of bm x bn tiles takes, in us per 4096 of K: the time of its busiest CU,
+// which runs r = ceil(tiles / CUs) of them, from launches timed on MI355X (gfx950, 256
+// CUs) after 100 ms of warm-up.  K itself scales all alike (measured down to K = 128).
+//   32 x 32:   26 alone on its CU, then 18.4 r (16 x 4096: 25.7; 480 x 816: 35 at r = 2;
+//              1000 x 1024: 69 .. 73 at r = 4; 2602 x 1960: 364 .. 382 at r = 20).
+//   32 x 64:   40 alone, then 34.5 r (1500 x 1000: 118 at r = 3; 1531 x 1021: 108 at r = 3;
+//              2048 x 2048: 270 at r = 8; 4096 x 4096: 1077 at r = 32).
+//   64 x 64:   69 alone, then 64.5 r (1024 x 1024: 67 .. 77; 1531 x 1021: 128 at r = 2;
+//              1000 x 4096: 261 at r = 4; 3000 x 4096: 762 at r = 12).
+//   128 x 64:  130 alone, then 10 + 122 r (1000 x 4096: 258 at r = 2; 2000 x 3000: 387 at
+//              r = 3; 3000 x 4096: 732 at r = 6; 4096 x 4096: 954 at r = 8).
+//   128 x 128: 257 alone, then 240 r, two tiles at a time: an odd last one shares its CU
+//              with nothing, or falls to a CU that has two (r = 3: 755 .. 949, so r + 0.6).
+//              2048 x 2048: 247 .. 269, 2048 x 4096: 511, 4096 x 4096: 937 .. 956.
+//   256 x 256: 950 r, one at a time (4096 x 4096: 926 .. 974).
+double tile_us(int bm, int bn, int64_t m, int64_t n, int64_t cus) {
+  const int64_t tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+  const double r = static_cast<double>(tiles > cus ? (tiles + cus - 1) / cus : 1);
+  const bool alone = tiles <= cus;
+  switch (bm * bn) {
+    case 32 * 32: return alone ? 26.0 : 18.4 * r;
+    case 32 * 64: return alone ? 40.0 : 34.5 * r;
+    case 64 * 64: return alone ? 69.0 : 64.5 * r;
+    case 128 * 64: return alone ? 130.0 : 10.0 + 122.0 * r;
+    case 128 * 128:
+      return alone ? 257.0 : 240.0 * (r + (static_cast<int64_t>(r) % 2 == 1 ? 0.6 : 0.0));
+    default: return 950.0 * r;
+  }
+}
+
 const MfmaCfg* find_mfma(const mcke_gemm_tile& t) {
   for (const MfmaCfg& c : kMfmaCfgs)
     if (tile_eq(t, c.bm, c.bn, c.bk, c.bm / 16, c.bn / 16)) return &c;
@@ -467,6 +517,25 @@ RowsPick find_rows(int64_t m, int64_t n, int64_t k, bool fused) {
   return p;
 }
 
+// The register-staged kernel at the requested tile: any shape and alignment.
+int launch_mfma_staged(const char* who, const Spec& sp, bool fused, const float* a, const float* b,
+                       float* c, int64_t m, int64_t n, int64_t k, float alpha, float beta,
+                       EpiArgs epi, hipStream_t s) {
+  const int64_t tiles_m = (m + sp.tile_m - 1) / sp.tile_m;
+  const int64_t tiles_n = (n + sp.tile_n - 1) / sp.tile_n;
+  if (tiles_m * tiles_n > 2147483647LL)
+    return invalid(std::string(who) + ": too many tiles for one launch");
+  if (tiles_m * tiles_n * static_cast<int64_t>(sp.block.x) > int64_t{UINT32_MAX})
+    return invalid(std::string(who) + ": tiles x lanes exceed the grid's 32-bit work size; use a "
+                   "larger tile");
+  MfmaFn fn = fused ? sp.mfma_f : sp.mfma;
+  fn<<<static_cast<unsigned>(tiles_m * tiles_n), sp.block, 0, s>>>(
+      a, b, c, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), alpha, beta,
+      static_cast<int>(tiles_m), static_cast<int>(tiles_n), epi);
+  MCKE_LAUNCH_CHECK(fused ? "gemm_mfma_kernel (bias + activation)" : "gemm_mfma_kernel");
+  return ok();
+}
+
 // One kMfmaF32 launch: few tiles of 32 x 32 take the few-tiles kernel, whole tiles
 // the direct-to-LDS kernel, and other shapes its EDGE form where a tile's columns fit in a
 // row of B and K holds a stage, else the staged kernel; `fused` picks the instantiations
@@ -487,19 +556,35 @@ int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, con
       return ok();
     }
   }
-  const int64_t tiles_m = (m + sp.tile_m - 1) / sp.tile_m;
-  const int64_t tiles_n = (n + sp.tile_n - 1) / sp.tile_n;
+  int bm = sp.tile_m, bn = sp.tile_n;
+  MfmaFn even = fused ? sp.mfma_even_f : sp.mfma_even;
+  MfmaFn edge = fused ? sp.mfma_edge_f : sp.mfma_edge;
+  if (bm == 64 && edge && floats && n >= 64 && k >= 32) {
+    const int64_t cus = device_cu_count();
+    double best = tile_us(64, 64, m, n, cus);
+    for (const SubTile& t : kSubTiles64) {
+      const double us = tile_us(t.bm, t.bn, m, n, cus);
+      if (us >= best || t.bm * k >= (int64_t{1} << 30)) continue;
+      best = us;
+      bm = t.bm;
+      bn = t.bn;
+      even = !even ? nullptr : fused ? t.even_f : t.even;
+      edge = fused ? t.edge_f : t.edge;
+    }
+  }
+  const int64_t tiles_m = (m + bm - 1) / bm;
+  const int64_t tiles_n = (n + bn - 1) / bn;
   if (tiles_m * tiles_n > 2147483647LL)
     return invalid(std::string(who) + ": too many tiles for one launch");
-  const bool offsets32 = static_cast<int64_t>(sp.tile_m) * k < (int64_t{1} << 30) &&
+  const bool offsets32 = static_cast<int64_t>(bm) * k < (int64_t{1} << 30) &&
                          static_cast<int64_t>(32) * n < (int64_t{1} << 30);
-  const bool whole = sp.mfma_even && m % sp.tile_m == 0 && n % sp.tile_n == 0 &&
-                     k % sp.tile_k == 0 && (!sp.even_dma || offsets32);
-  const bool edge = !whole && sp.mfma_edge && n >= sp.tile_n && k >= 32 && offsets32 && floats;
-  MfmaFn fn = fused ? (whole ? sp.mfma_even_f : edge ? sp.mfma_edge_f : sp.mfma_f)
-                    : (whole ? sp.mfma_even : edge ? sp.mfma_edge : sp.mfma);
-  const dim3 block =
-      whole || edge ? dim3(static_cast<unsigned>(sp.even_threads), 1, 1) : sp.block;
+  const bool whole = even && m % bm == 0 && n % bn == 0 && k % sp.tile_k == 0 &&
+                     (!sp.even_dma || offsets32);
+  const bool ragged = !whole && edge && n >= bn && k >= 32 && offsets32 && floats;
+  if (!whole && !ragged)
+    return launch_mfma_staged(who, sp, fused, a, b, c, m, n, k, alpha, beta, epi, s);
+  MfmaFn fn = whole ? even : edge;
+  const dim3 block(static_cast<unsigned>(sp.even_threads), 1, 1);
   if (tiles_m * tiles_n * static_cast<int64_t>(block.x) > int64_t{UINT32_MAX})
     return invalid(std::string(who) + ": tiles x lanes exceed the grid's 32-bit work size; use a "
                    "larger tile");
@@ -628,38 +713,21 @@ int mcke_launch_gemm_lp_vendor(const void* a, const void* b, void* c, int ab_dty
 
 int mcke_gemm_mfma_default_tile(int64_t m, int64_t n, int64_t k, mcke_gemm_tile* out) {
   if (!out) return invalid("gemm_mfma_default_tile: null out");
-  // What decides is how evenly a tile size fills the CUs: a launch takes as long as its
-  // busiest CU, which runs r = ceil(tiles / CUs) tiles.  Each candidate's cost is that
-  // CU's time, in us per 4096 of K, from launches timed on MI355X (gfx950, 256 CUs), and
-  // the lowest one wins (ties: the larger tile).  K itself scales all alike (measured
-  // down to K = 128).
-  //   32:  26 alone on its CU, then 18.4 r (16 x 4096: 25.7; 480 x 816: 37 at r = 2;
-  //        1000 x 1024: 73 at r = 4; 2602 x 1960: 364 at r = 20).
-  //   64:  73 alone, then 64.5 r (1024 x 1024: 75; 1531 x 1021: 132 at r = 2; 1000 x 4096:
-  //        261 at r = 4; 3000 x 4096: 788 at r = 12).
-  //   128: 257 alone, then 240 r, two tiles at a time: an odd last one shares its CU with
-  //        nothing, or falls to a CU that has two (r = 3: 755 .. 949, so r + 0.6).
-  //        2048 x 2048: 257 .. 269, 2048 x 4096: 511, 4096 x 4096 : 956.
-  //   256: 950 r, one at a time (4096 x 4096: 926 .. 974).
-  // Shapes that are not whole tiles cost the two large tiles 3% more (the EDGE form's
-  // row and column checks: 1000 x 4096 x 1024 69.8 us against 68.0 for 1024 rows).
-  struct Cand { int t; double alone, each; mcke_gemm_tile tile; };
-  static const Cand cands[] = {{256, 950.0, 950.0, {256, 256, 32, 16, 16}},
-                               {128, 257.0, 240.0, {128, 128, 32, 8, 8}},
-                               {64, 73.0, 64.5, {64, 64, 32, 4, 4}},
-                               {32, 26.0, 18.4, {32, 32, 32, 2, 2}}};
+  // The tile whose launch is the shortest (tile_us), ties to the larger one; the 64 x 64
+  // tile counts as the better of its own and the 32 x 64 one that it may run.  Shapes that
+  // are not whole tiles cost the two large tiles 3% more (the EDGE form's row and column
+  // checks: 1000 x 4096 x 1024 69.8 us against 68.0 for 1024 rows at 128 x 128).
+  static const mcke_gemm_tile cands[] = {
+      {256, 256, 32, 16, 16}, {128, 128, 32, 8, 8}, {64, 64, 32, 4, 4}, {32, 32, 32, 2, 2}};
   const int64_t cus = device_cu_count();
   double best = 0.0;
-  for (const Cand& c : cands) {
-    const int64_t tiles = ((m + c.t - 1) / c.t) * ((n + c.t - 1) / c.t);
-    const int64_t r = tiles > 0 ? (tiles + cus - 1) / cus : 1;
-    double cost = c.each * static_cast<double>(r);
-    if (r == 1) cost = c.alone;
-    else if (c.t == 128 && r % 2 == 1) cost += 0.6 * c.each;
-    if (c.t >= 128 && (m % c.t != 0 || n % c.t != 0 || k % 32 != 0)) cost *= 1.03;
-    if (c.t == 256 || cost < best) {
-      best = cost;
-      *out = c.tile;
+  for (const mcke_gemm_tile& c : cands) {
+    double us = tile_us(c.bm, c.bn, m, n, cus);
+    if (c.bm == 64) us = std::min(us, tile_us(32, 64, m, n, cus));
+    if (c.bm >= 128 && (m % c.bm != 0 || n % c.bn != 0 || k % 32 != 0)) us *= 1.03;
+    if (c.bm == 256 || us < best) {
+      best = us;
+      *out = c;
     }
   }
   return ok();

@@ -52,6 +52,44 @@ def test_gemm_f32_tile_edges(gpu, orc, t):
             del da, db
 
 
+# 64 x 64 launches that run 128 x 64 tiles (1000 x 4096: four 64 x 64 tiles per CU) and
+# 32 x 64 tiles (1531 x 1021: 1.5 per CU), whole and not.
+@pytest.mark.parametrize("shape", [(1024, 4096, 64), (1000, 4093, 70), (901, 4096, 33),
+                                   (1536, 1024, 96), (1531, 1021, 70), (1505, 1089, 32)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_64_tile_launch_picks(gpu, orc, shape):
+    M, N, K = shape
+    V, tile = gpu.GemmVariant.kMfmaF32, _tile(gpu, 64)
+    a = orc.fill_random(M * K, 61 + K).reshape(M, K)
+    b = orc.fill_random(K * N, 62 + N).reshape(K, N)
+    c = orc.fill_random(M * N, 63 + M).reshape(M, N)
+    bias = orc.fill_random(N, 64)
+    prod = a.astype(np.float64) @ b.astype(np.float64)
+    for sa, sb, sc, beta in ((0, 0, 0, 0.0), (1, 3, 2, 1.5)):
+        da, pa = _up(gpu, a, sa)
+        db, pb = _up(gpu, b, sb)
+        out = _Out(gpu, M * N, sc)
+        full = out.buf.download()
+        full[out.at:out.at + M * N] = np.nan if beta == 0.0 else c.ravel()
+        out.buf.upload(full)
+        st = gpu.launch_gemm_f32(pa, pb, out.ptr, M, N, K, 0.75, beta, V, tile)
+        assert st.ok(), str(st)
+        gpu.device_synchronize()
+        r = orc.compare(out.get(), (0.75 * prod + beta * c).ravel(), orc.tol_gemm(K),
+                        orc.abs_tol_gemm(K) + 4e-7)
+        assert r.ok, f"shifts={sa},{sb},{sc}: {r}"
+        if beta == 0.0:
+            dbias, pbias = _up(gpu, bias, 0)
+            y, fused = _Out(gpu, M * N, 0), _Out(gpu, M * N, 0)
+            for st in (gpu.launch_bias_act_f32(out.ptr, pbias, y.ptr, M, N, 3, 1),
+                       gpu.launch_gemm_bias_act_f32(pa, pb, pbias, fused.ptr, M, N, K, 0.75, 3,
+                                                    tile)):
+                assert st.ok(), str(st)
+            gpu.device_synchronize()
+            assert np.array_equal(fused.get().view(np.uint32), y.get().view(np.uint32))
+        del da, db
+
+
 @pytest.mark.parametrize("t", TILES)
 @pytest.mark.parametrize("act", [0, 1, 2, 3])
 def test_fused_tile_edges_match_the_pair(gpu, orc, t, act):
