@@ -20,6 +20,7 @@
 
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -137,6 +138,19 @@ class ExecutionPlan {
   std::vector<std::vector<Tensor>> writes_;
   std::size_t arena_bytes_ = 0;
   std::size_t unshared_bytes_ = 0;
+
+  // Pinned memory that read_tensor() takes large results through, a chunk at a time:
+  // present when the graph has an output of kStagedReadBytes or more.
+  struct ReadStage {
+    static constexpr std::size_t kChunk = std::size_t{768} << 10;
+    static constexpr std::size_t kSlots = 2;
+    std::mutex busy;
+    char* pinned = nullptr;
+    std::vector<rt::Event> landed;   // per slot: its last copy has arrived
+    ~ReadStage();
+  };
+  static constexpr std::size_t kStagedReadBytes = std::size_t{2} << 20;
+  std::unique_ptr<ReadStage> read_stage_;
 };
 
 class GraphExecutor {
@@ -181,6 +195,9 @@ class GraphExecutor {
   }
   [[nodiscard]] StatusOr<Tensor> output(TensorId t) const;
   [[nodiscard]] StatusOr<Tensor> any_bound_tensor(TensorId t) const;
+  // Copies the first `bytes` of tensor t (any with a buffer) to host memory, behind what
+  // stream 0 has queued, and waits for every stream of the plan.
+  [[nodiscard]] Status read_tensor(TensorId t, void* host, std::size_t bytes);
   [[nodiscard]] Status collect_timings();
   [[nodiscard]] StatusOr<NumericsResult> validate_numerics(int repeats = 20);
   [[nodiscard]] const std::vector<NodeTiming>& node_timings() const noexcept { return node_timings_; }
@@ -196,6 +213,9 @@ class GraphExecutor {
   void drop_replay();
   [[nodiscard]] Status run_program();                // one eager iteration
   [[nodiscard]] Status refill_poison(rt::Stream& s0);
+  [[nodiscard]] Status make_read_stage();
+  [[nodiscard]] Status read_staged(ExecutionPlan::ReadStage& st, const Tensor& src, void* host,
+                                   std::size_t bytes, rt::Stream& s0);
   [[nodiscard]] Status launch(std::size_t i, rt::Stream& lane);   // scheduled node i's op
   [[nodiscard]] Status capture_lanes(void** out_exec);            // multi-stream capture
   struct GateOutcome;

@@ -297,6 +297,8 @@ int mcke_rt_malloc(void** out_ptr, size_t bytes);
 int mcke_rt_free(void* ptr);
 int mcke_rt_host_alloc(void** out_ptr, size_t bytes); /* pinned host memory */
 int mcke_rt_host_free(void* ptr);
+/* 1 when ptr is ordinary host memory: not pinned, managed or on a device. */
+int mcke_rt_pointer_is_pageable(const void* ptr, int* pageable);
 /* kind: 0 host->device, 1 device->host, 2 device->device, 3 default (unified VA). */
 int mcke_rt_memcpy_async(void* dst, const void* src, size_t bytes, int kind, void* stream);
 /* Refused (INVALID_ARGUMENT) while `stream` is being captured into a graph: a

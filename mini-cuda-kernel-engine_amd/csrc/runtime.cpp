@@ -355,7 +355,11 @@ int mcke_rt_host_alloc(void** out_ptr, size_t bytes) {
   *out_ptr = nullptr;
   if (bytes == 0) return ok();
   void* p = nullptr;
-  MCKE_HIP_TRY(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+  const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocDefault);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // recoverable: callers may go on without it
+    return hip_fail(e, "hipHostMalloc", __FILE__, __LINE__);
+  }
   *out_ptr = p;
   return ok();
 }
@@ -363,6 +367,15 @@ int mcke_rt_host_alloc(void** out_ptr, size_t bytes) {
 int mcke_rt_host_free(void* ptr) {
   if (!ptr) return ok();
   MCKE_HIP_TRY(hipHostFree(ptr));
+  return ok();
+}
+
+int mcke_rt_pointer_is_pageable(const void* ptr, int* pageable) {
+  if (!pageable) return invalid("mcke_rt_pointer_is_pageable: null out");
+  hipPointerAttribute_t at{};
+  const hipError_t e = hipPointerGetAttributes(&at, ptr);
+  if (e != hipSuccess) (void)hipGetLastError();  // some runtimes refuse unknown memory instead
+  *pageable = e == hipErrorInvalidValue || (e == hipSuccess && at.type == hipMemoryTypeUnregistered);
   return ok();
 }
 

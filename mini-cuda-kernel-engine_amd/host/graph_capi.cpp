@@ -245,11 +245,7 @@ int mcke_executor_is_captured(mcke_executor* e, int* out) {
 
 int mcke_executor_read_tensor(mcke_executor* e, uint32_t t, void* host, size_t bytes) {
   if (!e || !host) return bad("null argument");
-  auto tr = e->exec->any_bound_tensor(t);
-  if (!tr.ok()) return code(tr.status());
-  const auto& plan = e->exec->plan_ref();
-  if (int rc = code(tr->copy_to_host(host, bytes, plan.stream(0)))) return rc;
-  return code(e->exec->synchronize());
+  return code(e->exec->read_tensor(t, host, bytes));
 }
 
 int mcke_executor_plan_info(mcke_executor* e, mcke_plan_info* out) {
