@@ -86,8 +86,8 @@ int launch_split(const LpArgs& x) {
   return launch_split_as<T, OutT, 4, 4, 4>(x);
 }
 
-// The register-staged kernel at the requested tile: what is narrower than any other
-// kernel's tile, or past their 32-bit offsets or grids.
+// The register-staged kernel's checked forms at the requested tile: what is narrower than
+// any other kernel's tile, or past their 32-bit offsets or grids.
 template <typename T, typename OutT, int BM, int BN>
 int launch_staged(const LpArgs& x, bool vec) {
   const int64_t tiles = tile_count(x.m, x.n, BM, BN);
@@ -95,6 +95,18 @@ int launch_staged(const LpArgs& x, bool vec) {
   auto* fn = vec ? &gemm_lp_kernel<T, OutT, BM, BN, true, false>
                  : &gemm_lp_kernel<T, OutT, BM, BN, false, false>;
   fn<<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
+      x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + BM - 1) / BM,
+      (x.n + BN - 1) / BN);
+  MCKE_LAUNCH_CHECK("gemm_lp_kernel");
+  return ok();
+}
+
+// The WHOLE form.
+template <typename T, typename OutT, int BM, int BN>
+int launch_whole(const LpArgs& x) {
+  const int64_t tiles = tile_count(x.m, x.n, BM, BN);
+  if (int rc = check_grid(tiles, kMfmaThreads)) return rc;
+  gemm_lp_kernel<T, OutT, BM, BN, false, true><<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
       x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + BM - 1) / BM,
       (x.n + BN - 1) / BN);
   MCKE_LAUNCH_CHECK("gemm_lp_kernel");
@@ -119,6 +131,13 @@ template <int BM, int BN> bool edge_fits(const LpArgs& x) {
          aligned(x.b, 4) && aligned(x.c, 4) && dma_offsets32<BM, BN>(x.n, x.k);
 }
 
+// The register-staged kernel's WHOLE form at BM x BN, where the shape and the addresses
+// allow it.
+template <int BM, int BN, typename OutT> bool whole_fits(const LpArgs& x) {
+  return x.n >= BN && x.k >= 64 && aligned(x.a, 2) && aligned(x.b, 2) &&
+         aligned(x.c, sizeof(OutT));
+}
+
 template <typename T, typename OutT, int BM, int BN>
 struct LpTile {
   // Whole tiles run the requested tile's direct-to-LDS kernel (tiles of 128 and more).
@@ -126,8 +145,14 @@ struct LpTile {
   // where they nearly fill the CUs (fp16 to fp32: 2757 x 432 x 6080, 88 tiles of 128,
   // 49.9 us against 54.9 for split K; 1628 x 800 x 1110, 91 tiles, 17.2 against 18.2;
   // 300 x 520 x 1032, 15 tiles, 15.4 against 6; 4095 x 4094 x 4090, 256 tiles of 256,
-  // 130 us against 205 at 128), and otherwise the split-K kernel, which every 64 x 64
-  // launch takes.
+  // 130 us against 205 at 128).  Odd extents run the register-staged kernel's WHOLE form
+  // where its 128 x 128 tiles fill most of the CUs (a tile alone on its CU takes 1.3 us per
+  // 64 of K, so fewer lose to split K: 1531 x 1021 x 2053, 96 tiles, 44.3 us against 31.5;
+  // 1700 x 1701 x 1024, 196 tiles, 23.9 against 21.6; 4032 x 843 x 2744, 224 tiles, 54.0
+  // against 68.7; 1901 x 2001 x 511, 240 tiles, 20.3 against 30.4; 3001 x 2501 x 901, 480
+  // tiles, 32.8 against 57.1), at 256 x 256 from 192 such tiles on (4095^3 191 us against
+  // 229 at 128 and 395 for split K; 3500 x 3501 x 2001, 196 tiles, 98 against 102).  What is
+  // left takes the split-K kernel, as every 64 x 64 launch does.
   static int launch(const LpArgs& x, bool vec) {
     if constexpr (BN >= 128) {
       if (vec && x.m % BM == 0 && x.n % BN == 0 && x.k % 64 == 0 && x.k > 0 &&
@@ -142,6 +167,11 @@ struct LpTile {
           return launch_dma<T, OutT, 256, 256, true>(x);
       if (edge_fits<128, 128>(x) && tile_count(x.m, x.n, 128, 128) >= 80)
         return launch_dma<T, OutT, 128, 128, true>(x);
+      if constexpr (BM == 256)
+        if (whole_fits<256, 256, OutT>(x) && tile_count(x.m, x.n, 256, 256) >= 192)
+          return launch_whole<T, OutT, 256, 256>(x);
+      if (whole_fits<128, 128, OutT>(x) && tile_count(x.m, x.n, 128, 128) >= 208)
+        return launch_whole<T, OutT, 128, 128>(x);
     }
     // 16-bit values at 2-byte addresses, per-lane offsets below 4 GiB, and a grid that holds
     // 32 x 32 tiles of 512 lanes.

@@ -1,6 +1,7 @@
 // gemm_lp.hpp -- 16-bit-input GEMM on the CDNA4 matrix cores, fp32 accumulation.
 // Kernels: gemm_lp_kernel (any shape, register-staged, 32x32x16 MFMAs, the layout
-// described first below; products narrower than 32 columns take it),
+// described first below; large products of odd extents and those narrower than 32 columns
+// take it),
 // gemm_lp_dma_kernel (direct-to-LDS, 32x32x16; whole 128 x 128 tiles with K % 64 == 32),
 // gemm_lp_dma16_kernel (direct-to-LDS, 16x16x32; whole tiles with K % 64 == 0, and an
 // EDGE form for other even shapes), each described where it is defined, and
@@ -56,6 +57,8 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 // 16 bytes at any 4-byte address.
 typedef unsigned u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+// 16 bytes at any 2-byte address.
+typedef unsigned u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 constexpr int kLpBK = 64;            // K depth of one LDS stage (elements)
 constexpr int kLpRowBytes = 128;     // one LDS row: 64 16-bit values
@@ -98,11 +101,11 @@ __device__ __forceinline__ int lp_swz(int r) { return (r & 7) ^ ((r >> 3) & 7); 
 // row of length `len`; VEC: one 16-byte load (len % 8 == 0, p 16-byte aligned,
 // so the chunk is wholly in or out of range); else per-element loads.  Elements
 // outside [0, len) -- and the whole chunk when !in_row -- read as +0.
-template <bool VEC, bool EVEN>
+template <bool VEC>
 __device__ __forceinline__ u32x4 lp_load8(const uint16_t* __restrict__ p, int k, int len,
                                           bool in_row) {
   if constexpr (VEC) {
-    if (EVEN || (in_row && k < len)) return *reinterpret_cast<const u32x4*>(p);
+    if (in_row && k < len) return *reinterpret_cast<const u32x4*>(p);
     return u32x4{0u, 0u, 0u, 0u};
   } else {
     unsigned v[8];
@@ -140,25 +143,57 @@ struct LpStage {
     return w * WN + (nl % NT) * 32 + nl / NT;
   }
 
-  template <bool VEC, bool EVEN>
+  // WHOLE: all of the stage is in range in k and n, at any 2-byte alignment; rows past M
+  // repeat row M - 1.
+  template <bool VEC, bool WHOLE>
   static __device__ __forceinline__ void load_a(Regs& R, int i, const uint16_t* __restrict__ A,
                                                 int M, int K, int m0, int k0) {
     const int li = i * kThreads + static_cast<int>(threadIdx.x);
     const int row = li / 8, kc = li % 8;
     const int gm = m0 + row, gk = k0 + 8 * kc;
-    const uint16_t* p = A + static_cast<int64_t>(EVEN || gm < M ? gm : 0) * K + gk;
-    R.a[i] = lp_load8<VEC, EVEN>(p, gk, K, EVEN || gm < M);
+    if constexpr (WHOLE) {
+      R.a[i] = *reinterpret_cast<const u32x4_a2*>(
+          A + static_cast<int64_t>(gm < M ? gm : M - 1) * K + gk);
+    } else {
+      const uint16_t* p = A + static_cast<int64_t>(gm < M ? gm : 0) * K + gk;
+      R.a[i] = lp_load8<VEC>(p, gk, K, gm < M);
+    }
   }
 
-  template <bool VEC, bool EVEN>
+  template <bool VEC, bool WHOLE>
   static __device__ __forceinline__ void load_b(Regs& R, int i, const uint16_t* __restrict__ B,
                                                 int N, int K, int n0, int k0) {
     const int t = static_cast<int>(threadIdx.x);
     const int nb = t % kBGroups, kb = t / kBGroups;
     const int gk = k0 + kb * KR + i, gn = n0 + 8 * nb;
-    const bool in_k = EVEN || gk < K;
-    const uint16_t* p = B + static_cast<int64_t>(in_k ? gk : 0) * N + gn;
-    R.b[i] = lp_load8<VEC, EVEN>(p, gn, N, in_k);
+    if constexpr (WHOLE) {
+      R.b[i] = *reinterpret_cast<const u32x4_a2*>(B + static_cast<int64_t>(gk) * N + gn);
+    } else {
+      const bool in_k = gk < K;
+      const uint16_t* p = B + static_cast<int64_t>(in_k ? gk : 0) * N + gn;
+      R.b[i] = lp_load8<VEC>(p, gn, N, in_k);
+    }
+  }
+
+  // The first `rem` of K as a stage, zero-padded in both operands.
+  static __device__ __forceinline__ void load_rem(Regs& R, const uint16_t* __restrict__ A,
+                                                  const uint16_t* __restrict__ B, int M, int N,
+                                                  int K, int m0, int n0, int rem) {
+    const int t = static_cast<int>(threadIdx.x);
+#pragma unroll
+    for (int i = 0; i < kAChunks; ++i) {
+      const int row = (i * kThreads + t) / 8, kc = (i * kThreads + t) % 8;
+      const int gm = m0 + row < M ? m0 + row : M - 1;
+      R.a[i] = lp_load8<false>(A + static_cast<int64_t>(gm) * K + 8 * kc, 8 * kc, rem, true);
+    }
+#pragma unroll
+    for (int i = 0; i < KR; ++i) {
+      const int gk = (t / kBGroups) * KR + i;
+      R.b[i] = u32x4{0u, 0u, 0u, 0u};
+      if (gk < rem)
+        R.b[i] = *reinterpret_cast<const u32x4_a2*>(B + static_cast<int64_t>(gk) * N + n0 +
+                                                    8 * (t % kBGroups));
+    }
   }
 
   static __device__ __forceinline__ void store_a(const Regs& R, int i, char* stage) {
@@ -194,17 +229,18 @@ struct LpStage {
 
 // Epilogue: C = alpha * acc + beta * C (C not read when beta == 0).  VEC: C rows
 // are 16-byte aligned when N % NT == 0, so a lane's NT adjacent outputs go out as
-// one store.
-template <typename OutT, int BM, int BN, bool VEC>
+// one store; WHOLE: at any address, columns from n_first on.
+template <typename OutT, int BM, int BN, bool VEC, bool WHOLE>
 __device__ __forceinline__ void lp_store_c(const f32x16 (&acc)[BM / 64][BN / 64],
                                            OutT* __restrict__ C, int M, int N, int m0, int n0,
-                                           int wm, int wn, int h, int c, float alpha,
+                                           int n_first, int wm, int wn, int h, int c, float alpha,
                                            float beta) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int MT = WM / 32, NT = WN / 32;
   using O = LpOut<OutT>;
   const int col0 = n0 + wn * WN + NT * c;
-  const bool vec_store = VEC && (N % NT == 0) && col0 + NT - 1 < N;
+  const bool vec_store =
+      WHOLE ? col0 >= n_first : VEC && (N % NT == 0) && col0 + NT - 1 < N;
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
 #pragma unroll
@@ -213,7 +249,7 @@ __device__ __forceinline__ void lp_store_c(const f32x16 (&acc)[BM / 64][BN / 64]
       if (row >= M) continue;
       OutT* crow = C + static_cast<int64_t>(row) * N;
       if (vec_store) {
-        struct alignas(NT * sizeof(OutT)) Pack { OutT v[NT]; };
+        struct alignas(WHOLE ? sizeof(OutT) : NT * sizeof(OutT)) Pack { OutT v[NT]; };
         Pack o;
         if (beta != 0.0f) {
           const Pack old = *reinterpret_cast<const Pack*>(crow + col0);
@@ -229,7 +265,7 @@ __device__ __forceinline__ void lp_store_c(const f32x16 (&acc)[BM / 64][BN / 64]
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
           const int col = col0 + j;
-          if (col < N) {
+          if (WHOLE ? col >= n_first : col < N) {
             float v = alpha * acc[i][j][r];
             if (beta != 0.0f) v += beta * O::to_f32(crow[col]);
             crow[col] = O::from_f32(v);
@@ -240,16 +276,21 @@ __device__ __forceinline__ void lp_store_c(const f32x16 (&acc)[BM / 64][BN / 64]
   }
 }
 
-// VEC: K % 8 == 0, N % 8 == 0, A/B/C 16-byte aligned.  EVEN: additionally M, N, K
-// multiples of the tile (no bounds checks at all).
-template <typename T, typename OutT, int BM, int BN, bool VEC, bool EVEN>
+// VEC: K % 8 == 0, N % 8 == 0, A/B/C 16-byte aligned; else any shape, two bytes at a time.
+// WHOLE: any M, any N >= BN, any K >= 64, 2-byte alignment, all loads of the loop 16 bytes
+// and unchecked: rows past M repeat row M - 1 and are not stored, the last tile column
+// starts at N - BN and stores only the columns of its own, and the first stage is K % 64,
+// zero-padded.  Bound by its operand loads and their way through registers into LDS (about
+// 14 bytes per clock and CU at 128 x 128); each operand is read half as often as by 64 x 64
+// tiles, which is what it gains on the split-K kernel: 4095 x 4095 x 1023, fp16 to fp32, 136
+// -> 65.6 us (524 TFLOP/s).
+template <typename T, typename OutT, int BM, int BN, bool VEC, bool WHOLE>
 __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, OutT* __restrict__ C,
     int M, int N, int K, float alpha, float beta, int tiles_m, int tiles_n) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int MT = WM / 32, NT = WN / 32;
   static_assert(MT >= 1 && (NT == 1 || NT == 2 || NT == 4), "unsupported wave tile");
-  static_assert(!EVEN || VEC, "whole tiles take the 16-byte path");
   using S = LpStage<BM, BN>;
   using MF = LpMfma<T>;
 
@@ -257,7 +298,8 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
 
   int tm, tn;
   mfma_tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * BM, n_first = tn * BN;
+  const int n0 = WHOLE && n_first > N - BN ? N - BN : n_first;
 
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
@@ -273,13 +315,20 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
   const int ksteps = (K + kLpBK - 1) / kLpBK;
+  // Stage s > 0 starts at k = 64 s - k_short.
+  const int rem = WHOLE ? K % kLpBK : 0;
+  const int k_short = rem ? kLpBK - rem : 0;
   typename S::Regs R;
   if (ksteps > 0) {
+    if (rem) {
+      S::load_rem(R, A, B, M, N, K, m0, n0, rem);
+    } else {
 #pragma unroll
-    for (int i = 0; i < S::kAChunks; ++i)
-      S::template load_a<VEC, EVEN>(R, i, A, M, K, m0, 0);
+      for (int i = 0; i < S::kAChunks; ++i)
+        S::template load_a<VEC, WHOLE>(R, i, A, M, K, m0, 0);
 #pragma unroll
-    for (int i = 0; i < S::KR; ++i) S::template load_b<VEC, EVEN>(R, i, B, N, K, n0, 0);
+      for (int i = 0; i < S::KR; ++i) S::template load_b<VEC, WHOLE>(R, i, B, N, K, n0, 0);
+    }
 #pragma unroll
     for (int i = 0; i < S::kAChunks; ++i) S::store_a(R, i, smem);
     S::store_b(R, smem);
@@ -308,8 +357,9 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
     char* next_stage = smem + ((ks + 1) & 1) * S::kBytes;
     const bool more = (ks + 1) < ksteps;
     // The last step re-loads itself (k clamped) into the unused buffer: harmless,
-    // and it keeps the loop free of branches around the loads.
-    const int k_next = (more ? ks + 1 : ks) * kLpBK;
+    // and it keeps the loop free of branches around the loads.  (WHOLE: with K >= 64 the
+    // last stage is never the remainder.)
+    const int k_next = (more ? ks + 1 : ks) * kLpBK - k_short;
 
     u32x4 av[MT], bv[NT], av_n[MT], bv_n[NT];
 #pragma unroll
@@ -334,8 +384,8 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
 #pragma unroll
       for (int l = 0; l < kLoads; ++l) {
         if ((2 * l) / kLoads == s) {
-          if (l < S::kAChunks) S::template load_a<VEC, EVEN>(R, l, A, M, K, m0, k_next);
-          else S::template load_b<VEC, EVEN>(R, l - S::kAChunks, B, N, K, n0, k_next);
+          if (l < S::kAChunks) S::template load_a<VEC, WHOLE>(R, l, A, M, K, m0, k_next);
+          else S::template load_b<VEC, WHOLE>(R, l - S::kAChunks, B, N, K, n0, k_next);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -364,7 +414,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
     __syncthreads();
   }
 
-  lp_store_c<OutT, BM, BN, VEC>(acc, C, M, N, m0, n0, wm, wn, h, c, alpha, beta);
+  lp_store_c<OutT, BM, BN, VEC, WHOLE>(acc, C, M, N, m0, n0, n_first, wm, wn, h, c, alpha, beta);
 }
 
 // ---------------------------------------------------------------------------

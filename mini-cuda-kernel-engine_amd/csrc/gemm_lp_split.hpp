@@ -36,8 +36,6 @@
 namespace mcke_amd {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-// 16 bytes at any 2-byte address.
-typedef unsigned u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 template <int MT, int NW, int WV, int H>
 struct LpSplitShape {

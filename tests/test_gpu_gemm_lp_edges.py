@@ -1,6 +1,7 @@
 """GPU parity of the 16-bit GEMM at shapes that are not whole tiles: the EDGE form of the
-direct-to-LDS kernel and the split-K kernel, around their tiles, K steps and limits, with
-operands and C at every element offset, C between guard values that must keep their bits.
+direct-to-LDS kernel, the WHOLE form of the register-staged one and the split-K kernel,
+around their tiles, K steps and limits, with operands and C at every element offset, C
+between guard values that must keep their bits.
 
 Bars: quarter-multiple inputs make every sum exact in fp32, so the result is the oracle's
 bit for bit; infinities and NaN reach their own outputs only.
@@ -21,6 +22,12 @@ GUARD = 16
 EDGE_128 = [(1279, 1024, 64), (1151, 1150, 66), (1025, 1154, 94), (10200, 130, 160),
             (129, 10112, 126)]
 EDGE_256 = [(3073, 4000, 66), (3100, 4098, 128)]
+# The register-staged kernel's WHOLE form: odd N or K, from 208 tiles of 128 or 192 of 256
+# on; K % 64 of 0, 1, 32, 63 as the first stage, one and two stages, last tile columns of 1
+# and 127 columns of their own.
+WHOLE_128 = [(1921, 1665, 64), (1793, 1919, 65), (1665, 2049, 191), (13300, 129, 96),
+             (129, 13311, 127), (1409, 2563, 321)]
+WHOLE_256 = [(3073, 3841, 66), (3100, 4095, 127)]
 # Split K: 16 and 32 rows (8 waves), 32 x 64 and 64 x 64 tiles (past 1024 of 32 x 64), odd
 # widths, K around its 32-deep chunks dealt to 4 and 8 waves; N below 32: register-staged.
 SPLIT = [(1, 32, 1), (16, 33, 31), (15, 8191, 33), (17, 100, 257), (32, 63, 256), (33, 63, 96),
@@ -78,6 +85,15 @@ def test_edge_tiles(gpu, orc, dt, out, shape):
 
 @pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
 @pytest.mark.parametrize("out", ["f32", "same"])
+@pytest.mark.parametrize("shape", WHOLE_128 + WHOLE_256, ids=lambda s: "x".join(map(str, s)))
+def test_whole_form_of_the_staged_kernel(gpu, orc, dt, out, shape):
+    tile = gpu.LP_TILES[0] if shape in WHOLE_256 else gpu.LP_TILES[1]
+    _check(gpu, orc, dt, out, *shape, tile, (0, 0, 0), 1.0, 0.0)
+    _check(gpu, orc, dt, out, *shape, tile, (1, 3, 1), 0.5, 2.0)
+
+
+@pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
+@pytest.mark.parametrize("out", ["f32", "same"])
 @pytest.mark.parametrize("shape", SPLIT, ids=lambda s: "x".join(map(str, s)))
 def test_split_k(gpu, orc, dt, out, shape):
     _check(gpu, orc, dt, out, *shape, gpu.LP_TILES[2], (0, 0, 0), 1.0, 0.0)
@@ -87,7 +103,8 @@ def test_split_k(gpu, orc, dt, out, shape):
 def test_remainders_keep_special_values_apart(gpu, orc):
     """The K remainder pads both operands with zeros: infinities and NaN in the last columns
     of A and the last rows of B reach their own outputs only."""
-    for M, N, K, tile in ((1279, 1026, 70, gpu.LP_TILES[1]), (37, 131, 45, gpu.LP_TILES[2])):
+    for M, N, K, tile in ((1279, 1026, 70, gpu.LP_TILES[1]),
+                          (1921, 1665, 131, gpu.LP_TILES[1]), (37, 131, 45, gpu.LP_TILES[2])):
         rng = np.random.default_rng(K)
         a, b = _quarters(rng, (M, K)), _quarters(rng, (K, N))
         a[M - 1, 3], a[0, K - 1] = np.nan, np.inf
