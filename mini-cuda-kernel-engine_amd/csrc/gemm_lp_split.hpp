@@ -2,7 +2,7 @@
 // row-major, bf16 or fp16 in, fp32 accumulation, fp32 or 16-bit C; any M, any N >= the
 // tile's width, any K, any element alignment.
 //
-// For tiles up to 64 x 64 and for shapes the direct-to-LDS kernels do not take.  With a
+// For tiles up to 64 x 64 and for shapes that fill too few CUs with larger ones.  With a
 // tile this small a 2 x 2 wave grid reads each operand from LDS twice (256 bytes per
 // cycle at 64 x 64 for 16x16x32 MFMAs, twice what LDS delivers) and meets at a barrier
 // for a few MFMAs' worth of work.  Here
