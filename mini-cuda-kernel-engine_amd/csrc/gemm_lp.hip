@@ -27,8 +27,15 @@ bool dma_offsets32(int n, int k) {
          static_cast<int64_t>(64) * n * 2 < (int64_t{1} << 32);
 }
 
+// Tiles along one extent.  Extents go up to INT32_MAX, where extent + tile - 1 does not fit
+// an int.
+constexpr int tiles_along(int extent, int tile) {
+  return static_cast<int>((static_cast<int64_t>(extent) + tile - 1) / tile);
+}
+static_assert(tiles_along(INT32_MAX, 256) == 1 << 23 && tiles_along(1, 256) == 1);
+
 int64_t tile_count(int m, int n, int bm, int bn) {
-  return ((static_cast<int64_t>(m) + bm - 1) / bm) * ((static_cast<int64_t>(n) + bn - 1) / bn);
+  return static_cast<int64_t>(tiles_along(m, bm)) * tiles_along(n, bn);
 }
 
 struct LpArgs {
@@ -53,8 +60,8 @@ int launch_dma(const LpArgs& x) {
   if (int rc = check_grid(tiles, kMfmaThreads)) return rc;
   gemm_lp_dma16_kernel<T, OutT, BM, BN, EDGE>
       <<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
-          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + BM - 1) / BM,
-          (x.n + BN - 1) / BN);
+          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
+          tiles_along(x.m, BM), tiles_along(x.n, BN));
   MCKE_LAUNCH_CHECK("gemm_lp_dma16_kernel");
   return ok();
 }
@@ -66,8 +73,8 @@ int launch_split_as(const LpArgs& x) {
   if (int rc = check_grid(tiles, WV * kWave)) return rc;
   gemm_lp_split_kernel<T, OutT, MT, NW, WV, 1>
       <<<static_cast<unsigned>(tiles), WV * kWave, 0, x.s>>>(
-          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + TM - 1) / TM,
-          (x.n + TN - 1) / TN);
+          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
+          tiles_along(x.m, TM), tiles_along(x.n, TN));
   MCKE_LAUNCH_CHECK("gemm_lp_split_kernel");
   return ok();
 }
@@ -95,8 +102,8 @@ int launch_staged(const LpArgs& x, bool vec) {
   auto* fn = vec ? &gemm_lp_kernel<T, OutT, BM, BN, true, false>
                  : &gemm_lp_kernel<T, OutT, BM, BN, false, false>;
   fn<<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
-      x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + BM - 1) / BM,
-      (x.n + BN - 1) / BN);
+      x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
+      tiles_along(x.m, BM), tiles_along(x.n, BN));
   MCKE_LAUNCH_CHECK("gemm_lp_kernel");
   return ok();
 }
@@ -107,8 +114,8 @@ int launch_whole(const LpArgs& x) {
   const int64_t tiles = tile_count(x.m, x.n, BM, BN);
   if (int rc = check_grid(tiles, kMfmaThreads)) return rc;
   gemm_lp_kernel<T, OutT, BM, BN, false, true><<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
-      x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta, (x.m + BM - 1) / BM,
-      (x.n + BN - 1) / BN);
+      x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
+      tiles_along(x.m, BM), tiles_along(x.n, BN));
   MCKE_LAUNCH_CHECK("gemm_lp_kernel");
   return ok();
 }

@@ -123,3 +123,41 @@ def test_remainders_keep_special_values_apart(gpu, orc):
         assert np.array_equal(np.isnan(got), np.isnan(want))
         ok = ~np.isnan(want)
         assert np.array_equal(got[ok], want[ok])
+
+
+@pytest.mark.parametrize("along", ["rows", "columns"])
+def test_extents_up_to_int32_max(gpu, orc, along):
+    """INT32_MAX rows or columns are accepted (extent + tile - 1 is past an int there): an
+    outer product with one column or row, whose every value is half the long operand's."""
+    n, period = 2**31 - 1, 1000003
+    M, N = (n, 1) if along == "rows" else (1, n)
+    tile = gpu.gemm_lp_default_tile(M, N, 1)
+    pattern = orc.to_16(((np.arange(period) * 7) % 1021 / 4.0).astype(np.float32), F16)
+    want = orc.to_16(orc.from_16(pattern, F16) * np.float32(0.5), F16)
+    copy = gpu.lib().mcke_rt_memcpy_async
+    x, y = gpu.DeviceBuffer(2 * n), gpu.DeviceBuffer(2 * (n + GUARD))
+    half = gpu.DeviceBuffer.from_array(orc.to_16(np.full(1, 0.5, np.float32), F16))
+    head = gpu.DeviceBuffer.from_array(pattern)
+    assert copy(x.ptr, head.ptr, 2 * period, 2, None) == 0
+    done = 2 * period
+    while done < 2 * n:                     # the part that is there, again behind itself
+        take = min(done, 2 * n - done)
+        assert copy(x.ptr + done, x.ptr, take, 2, None) == 0
+        done += take
+    mark = gpu.DeviceBuffer.from_array(np.full(GUARD, 77, np.uint16))
+    assert copy(y.ptr + 2 * n, mark.ptr, 2 * GUARD, 2, None) == 0
+    a, b = (x, half) if along == "rows" else (half, x)
+    st = gpu.launch_gemm_lp(a, b, y, F16, F16, M, N, 1, 1.0, 0.0, tile)
+    assert st.ok(), str(st)
+    gpu.device_synchronize()
+    chunk = np.empty(32 * period, np.uint16)
+    tiled = np.tile(want, 32)
+    for at in range(0, n, chunk.size):
+        part = chunk[:min(chunk.size, n - at)]
+        assert copy(part.ctypes.data, y.ptr + 2 * at, part.nbytes, 1, None) == 0
+        gpu.device_synchronize()
+        assert np.array_equal(part, tiled[:part.size]), f"in [{at}, {at + part.size})"
+    tail = np.empty(GUARD, np.uint16)
+    assert copy(tail.ctypes.data, y.ptr + 2 * n, tail.nbytes, 1, None) == 0
+    gpu.device_synchronize()
+    assert (tail == 77).all()
