@@ -29,10 +29,14 @@ WHOLE_128 = [(1921, 1665, 64), (1793, 1919, 65), (1665, 2049, 191), (13300, 129,
              (129, 13311, 127), (1409, 2563, 321)]
 WHOLE_256 = [(3073, 3841, 66), (3100, 4095, 127)]
 # Split K: 16 and 32 rows (8 waves), 32 x 64 and 64 x 64 tiles (past 1024 of 32 x 64), odd
-# widths, K around its 32-deep chunks dealt to 4 and 8 waves; N below 32: register-staged.
+# widths, K around its 32-deep chunks dealt to 4 and 8 waves, none and several to a wave; the
+# remainder with wave 0 or another, below 8, a multiple of 8 or not; N below 32:
+# register-staged.
 SPLIT = [(1, 32, 1), (16, 33, 31), (15, 8191, 33), (17, 100, 257), (32, 63, 256), (33, 63, 96),
          (33, 64, 32), (65, 131, 65), (200, 136, 264), (127, 1001, 127), (257, 9001, 63),
-         (5, 8193, 70), (3001, 1501, 35), (40, 31, 64), (7, 5, 3)]
+         (5, 8193, 70), (3001, 1501, 35), (40, 31, 64), (7, 5, 3), (33, 100, 7), (1, 64, 8),
+         (65, 131, 41), (16, 4096, 1031), (32, 515, 2049), (17, 8191, 545), (100, 63, 1100),
+         (70, 200, 1183), (2049, 2051, 271)]
 
 
 def _check(m, orc, dt, out, M, N, K, tile, shifts, alpha, beta):
