@@ -108,6 +108,24 @@ int launch_staged(const LpArgs& x, bool vec) {
   return ok();
 }
 
+// Short K over many tiles: the product is its C store, and the register-staged kernel's four
+// waves share a tile's one stage where the split-K kernel has one wave work and three add
+// zeros.  16-byte operands up to 63 of K (fp16 to fp32, 2460 x 1608 x 40: 7.6 us at 64 x 64
+// against 10.7 for split K; up to 1024 tiles they tie, 1101 x 1104 x 40 4.98 against 4.6),
+// others up to 7, as their loads are element by element (2460 x 1607 x 7: 10.2 against 11.1;
+// x 16: 11.8 against 9.9).  128 x 128 tiles where they fill two rounds of CUs or more to 80%
+// (2166 x 3544 x 40: 10.9 us against 12.1 at 64 x 64; 2460 x 1608, 260 tiles: 10.3 against 7.6).
+bool short_k(const LpArgs& x, bool vec) {
+  return x.k < (vec ? 64 : 8) && tile_count(x.m, x.n, 32, 64) > 1024;
+}
+
+template <typename T, typename OutT>
+int launch_short_k(const LpArgs& x, bool vec) {
+  const int64_t tiles = tile_count(x.m, x.n, 128, 128), rounds = (tiles + 255) / 256;
+  if (rounds >= 2 && 10 * tiles >= 8 * 256 * rounds) return launch_staged<T, OutT, 128, 128>(x, vec);
+  return launch_staged<T, OutT, 64, 64>(x, vec);
+}
+
 // The WHOLE form.
 template <typename T, typename OutT, int BM, int BN>
 int launch_whole(const LpArgs& x) {
@@ -148,10 +166,12 @@ template <int BM, int BN, typename OutT> bool whole_fits(const LpArgs& x) {
 template <typename T, typename OutT, int BM, int BN>
 struct LpTile {
   // Whole tiles run the requested tile's direct-to-LDS kernel (tiles of 128 and more).
-  // Other shapes run its EDGE form, at 128 x 128 from 80 such tiles on and at 256 x 256
+  // Other shapes run its EDGE form, at 128 x 128 from 208 such tiles on, or from 80 on where
+  // K is long enough to pay for a tile alone on its CU, and at 256 x 256
   // where they nearly fill the CUs (fp16 to fp32: 2757 x 432 x 6080, 88 tiles of 128,
   // 49.9 us against 54.9 for split K; 1628 x 800 x 1110, 91 tiles, 17.2 against 18.2;
-  // 300 x 520 x 1032, 15 tiles, 15.4 against 6; 4095 x 4094 x 4090, 256 tiles of 256,
+  // 300 x 520 x 1032, 15 tiles, 15.4 against 6; 4524 x 344 x 96, 108 tiles, 7.5 against 5.4,
+  // to fp16 5.6 against 5.1; 4095 x 4094 x 4090, 256 tiles of 256,
   // 130 us against 205 at 128).  Odd extents run the register-staged kernel's WHOLE form
   // where its 128 x 128 tiles fill most of the CUs (a tile alone on its CU takes 1.3 us per
   // 64 of K, so fewer lose to split K: 1531 x 1021 x 2053, 96 tiles, 44.3 us against 31.5;
@@ -172,20 +192,23 @@ struct LpTile {
       if constexpr (BM == 256)
         if (edge_fits<256, 256>(x) && tile_count(x.m, x.n, 256, 256) >= 192)
           return launch_dma<T, OutT, 256, 256, true>(x);
-      if (edge_fits<128, 128>(x) && tile_count(x.m, x.n, 128, 128) >= 80)
+      const int64_t tiles = tile_count(x.m, x.n, 128, 128);
+      if (edge_fits<128, 128>(x) &&
+          (tiles >= 208 || (tiles >= 80 && x.k >= (sizeof(OutT) == 4 ? 256 : 100))))
         return launch_dma<T, OutT, 128, 128, true>(x);
       if constexpr (BM == 256)
         if (whole_fits<256, 256, OutT>(x) && tile_count(x.m, x.n, 256, 256) >= 192)
           return launch_whole<T, OutT, 256, 256>(x);
-      if (whole_fits<128, 128, OutT>(x) && tile_count(x.m, x.n, 128, 128) >= 208)
+      if (whole_fits<128, 128, OutT>(x) && tiles >= 208)
         return launch_whole<T, OutT, 128, 128>(x);
     }
     // 16-bit values at 2-byte addresses, per-lane offsets below 4 GiB, and a grid that holds
     // 32 x 32 tiles of 512 lanes.
     if (x.n >= 32 && x.k > 0 && tile_count(x.m, x.n, 32, 32) <= int64_t{UINT32_MAX} / 512 &&
-        aligned(x.a, 2) && aligned(x.b, 2) && aligned(x.c, sizeof(OutT)) && static_cast<int64_t>(64) * x.k * 2 < (int64_t{1} << 32) &&
+        aligned(x.a, 2) && aligned(x.b, 2) && aligned(x.c, sizeof(OutT)) &&
+        static_cast<int64_t>(64) * x.k * 2 < (int64_t{1} << 32) &&
         static_cast<int64_t>(64) * x.n * 2 < (int64_t{1} << 32))
-      return launch_split<T, OutT>(x);
+      return short_k(x, vec) ? launch_short_k<T, OutT>(x, vec) : launch_split<T, OutT>(x);
     return launch_staged<T, OutT, BM, BN>(x, vec);
   }
   // The instantiation whole-tile shapes run, for attribute queries.

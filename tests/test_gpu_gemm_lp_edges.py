@@ -17,10 +17,12 @@ pytestmark = pytest.mark.gpu
 
 GUARD = 16
 
-# EDGE at 128 x 128 takes even N >= 128 and K >= 64 from 80 tiles on, at 256 x 256 from 192
+# EDGE at 128 x 128 takes even N >= 128 and K >= 64 from 208 tiles on (from 80 on where K is
+# at least 256, 100 with a 16-bit C; else the first five run split K), at 256 x 256 from 192
 # tiles on; K % 64 is its first pair of steps (0, 2, 30, 32, 62 left over).
 EDGE_128 = [(1279, 1024, 64), (1151, 1150, 66), (1025, 1154, 94), (10200, 130, 160),
-            (129, 10112, 126)]
+            (129, 10112, 126), (1663, 2048, 64), (1919, 1790, 66), (1665, 2050, 94),
+            (10200, 330, 160), (129, 13440, 126), (1151, 1150, 290)]
 EDGE_256 = [(3073, 4000, 66), (3100, 4098, 128)]
 # The register-staged kernel's WHOLE form: odd N or K, from 208 tiles of 128 or 192 of 256
 # on; K % 64 of 0, 1, 32, 63 as the first stage, one and two stages, last tile columns of 1
@@ -37,6 +39,12 @@ SPLIT = [(1, 32, 1), (16, 33, 31), (15, 8191, 33), (17, 100, 257), (32, 63, 256)
          (5, 8193, 70), (3001, 1501, 35), (40, 31, 64), (7, 5, 3), (33, 100, 7), (1, 64, 8),
          (65, 131, 41), (16, 4096, 1031), (32, 515, 2049), (17, 8191, 545), (100, 63, 1100),
          (70, 200, 1183), (2049, 2051, 271)]
+
+
+# Past 1024 tiles of 32 x 64, K below 64 where rows are 16-byte aligned and below 8 elsewhere:
+# the register-staged kernel, at 128 x 128 for the last two (441 and 476 tiles), else 64 x 64.
+SHORT_K = [(2081, 1032, 8), (2460, 1608, 56), (2293, 1737, 7), (4097, 513, 1), (2166, 3544, 40),
+           (2688, 2688, 56)]
 
 
 def _check(m, orc, dt, out, M, N, K, tile, shifts, alpha, beta):
@@ -104,10 +112,19 @@ def test_split_k(gpu, orc, dt, out, shape):
     _check(gpu, orc, dt, out, *shape, gpu.LP_TILES[2], (1, 3, 1), 0.5, 2.0)
 
 
+@pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
+@pytest.mark.parametrize("out", ["f32", "same"])
+@pytest.mark.parametrize("shape", SHORT_K, ids=lambda s: "x".join(map(str, s)))
+def test_short_k(gpu, orc, dt, out, shape):
+    tile = gpu.gemm_lp_default_tile(*shape)
+    _check(gpu, orc, dt, out, *shape, tile, (0, 0, 0), 1.0, 0.0)
+    _check(gpu, orc, dt, out, *shape, tile, (1, 3, 1), 0.5, 2.0)
+
+
 def test_remainders_keep_special_values_apart(gpu, orc):
     """The K remainder pads both operands with zeros: infinities and NaN in the last columns
     of A and the last rows of B reach their own outputs only."""
-    for M, N, K, tile in ((1279, 1026, 70, gpu.LP_TILES[1]),
+    for M, N, K, tile in ((1663, 2050, 70, gpu.LP_TILES[1]), (1279, 1026, 70, gpu.LP_TILES[1]),
                           (1921, 1665, 131, gpu.LP_TILES[1]), (37, 131, 45, gpu.LP_TILES[2])):
         rng = np.random.default_rng(K)
         a, b = _quarters(rng, (M, K)), _quarters(rng, (K, N))
