@@ -314,7 +314,8 @@ static_assert(kDmaThreads<128, 64, 1> == kMfmaThreads && kDmaThreads<32, 64, 2> 
 
 // What a launch of bm x bn tiles takes, in us per 4096 of K: the time of its busiest CU,
 // which runs r = ceil(tiles / CUs) of them, from launches timed on MI355X (gfx950, 256
-// CUs) after 100 ms of warm-up.  K itself scales all alike (measured down to K = 128).
+// CUs) after 100 ms of warm-up.  K itself scales all alike, down to about 256; below that a
+// tile's fixed cost shows (tile_fixed_us).
 //   32 x 32:   26 alone on its CU, then 18.4 r (16 x 4096: 25.7; 480 x 816: 35 at r = 2;
 //              1000 x 1024: 69 .. 73 at r = 4; 2602 x 1960: 364 .. 382 at r = 20).
 //   32 x 64:   40 alone, then 34.5 r (1500 x 1000: 118 at r = 3; 1531 x 1021: 108 at r = 3;
@@ -339,6 +340,22 @@ double tile_us(int bm, int bn, int64_t m, int64_t n, int64_t cus) {
     case 128 * 128:
       return alone ? 257.0 : 240.0 * (r + (static_cast<int64_t>(r) % 2 == 1 ? 0.6 : 0.0));
     default: return 950.0 * r;
+  }
+}
+
+// What a tile costs whatever its K: its prologue and its C store.  Fitted to launches of K 4
+// to 256 over 75 shapes (us: 32 x 32 0.45 .. 0.57 a tile, 32 x 64 0.44, 64 x 64 0.6 .. 1.4,
+// 128 x 128 2.1 .. 5).  Without it the smallest tile was taken for them: 576 x 3904 x 48
+// 11.2 us at 32 x 32 against 8.6 at 64 x 64, 4614 x 6836 x 16 52.4 at 128 x 128 against 46.9.
+double tile_fixed_us(int bm, int bn, int64_t m, int64_t n, int64_t cus) {
+  const int64_t tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+  const double r = static_cast<double>((tiles + cus - 1) / cus);
+  switch (bm * bn) {
+    case 32 * 32: return 0.4 * r;
+    case 32 * 64: return 0.5 * r;
+    case 64 * 64: return 0.8 * r;
+    case 128 * 128: return 4.0 * r;
+    default: return 16.0 * r;   // 256 x 256
   }
 }
 
@@ -488,7 +505,9 @@ using RowsFn = void (*)(const float*, const float*, float*, int, int, int, float
 // their sums: 16 x 32 ties at 7 x 6015 x 628 (7.4 us against 7.3 for the 32 x 32 tile) and
 // leads at 128 x 1012 x 320 (4.4 against 4.5); 32 x 32 leads from K = 1024 on (512 x 512 x
 // 1024: 7.7 against 8.7; 500 x 500 x 1000: 9.9 against 9.6); 16 x 64 trails at 16 x 16384 x
-// 256 (6.1 against 5.6) and leads at 16 x 16384 x 4096.  Per-lane source offsets are 32-bit.
+// 256 (6.1 against 5.6) and leads at 16 x 16384 x 4096.  K of 32 or less is one chunk, which
+// one of the eight waves works on: the 32 x 32 tile leads there by 0.1 .. 0.3 of 4.3 us.
+// Per-lane source offsets are 32-bit.
 struct RowsPick {
   RowsFn fn = nullptr;
   int tiles_m = 0, tiles_n = 0;
@@ -509,7 +528,7 @@ RowsPick find_rows(int64_t m, int64_t n, int64_t k, bool fused) {
     p.fn = fused ? &gemm_rows_kernel<MT, NW, true> : &gemm_rows_kernel<MT, NW, false>;        \
     return p;                                                                                 \
   }
-  MCKE_ROWS(1, 1, 1)
+  MCKE_ROWS(1, 1, 33)
   MCKE_ROWS(1, 2, 320)
   MCKE_ROWS(2, 2, 1024)
   if (m <= 16) MCKE_ROWS(1, 4, 1024)
@@ -538,7 +557,7 @@ int launch_mfma_staged(const char* who, const Spec& sp, bool fused, const float*
 
 // One kMfmaF32 launch: few tiles of 32 x 32 take the few-tiles kernel, whole tiles
 // the direct-to-LDS kernel, and other shapes its EDGE form where a tile's columns fit in a
-// row of B and K holds a stage, else the staged kernel; `fused` picks the instantiations
+// row of B and K is long enough, else the staged kernel; `fused` picks the instantiations
 // with the bias + activation epilogue, which route shapes exactly as the plain ones do
 // (so a fused launch accumulates in the plain launch's order).
 int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, const float* b,
@@ -559,12 +578,18 @@ int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, con
   int bm = sp.tile_m, bn = sp.tile_n;
   MfmaFn even = fused ? sp.mfma_even_f : sp.mfma_even;
   MfmaFn edge = fused ? sp.mfma_edge_f : sp.mfma_edge;
-  if (bm == 64 && edge && floats && n >= 64 && k >= 32) {
+  // EDGE from K = 64 on.  Below that most of K is the remainder, and the staged kernel is as
+  // fast or faster: 576 x 3904 x 40 8.5 us against 9.5, 4256 x 4864 x 40 40.1 against 46.8 at
+  // 64 x 64, 4416 x 288 x 32 unaligned 6.2 against 6.7 at 32 x 32.  Only where it loads 4 bytes
+  // at a time (`even` is null) do larger tiles gain from K = 32 on: 4614 x 6836 x 40 67 against 56.
+  const bool edge_k = k >= (bm >= 64 && !even ? 32 : 64);
+  if (bm == 64 && edge && floats && n >= 64 && (edge_k || (even && k == 32))) {
     const int64_t cus = device_cu_count();
     double best = tile_us(64, 64, m, n, cus);
     for (const SubTile& t : kSubTiles64) {
       const double us = tile_us(t.bm, t.bn, m, n, cus);
       if (us >= best || t.bm * k >= (int64_t{1} << 30)) continue;
+      if (!edge_k && (m % t.bm != 0 || n % t.bn != 0)) continue;
       best = us;
       bm = t.bm;
       bn = t.bn;
@@ -580,7 +605,7 @@ int launch_mfma(const char* who, const Spec& sp, bool fused, const float* a, con
                          static_cast<int64_t>(32) * n < (int64_t{1} << 30);
   const bool whole = even && m % bm == 0 && n % bn == 0 && k % sp.tile_k == 0 &&
                      (!sp.even_dma || offsets32);
-  const bool ragged = !whole && edge && n >= bn && k >= 32 && offsets32 && floats;
+  const bool ragged = !whole && edge && edge_k && n >= bn && offsets32 && floats;
   if (!whole && !ragged)
     return launch_mfma_staged(who, sp, fused, a, b, c, m, n, k, alpha, beta, epi, s);
   MfmaFn fn = whole ? even : edge;
@@ -713,17 +738,23 @@ int mcke_launch_gemm_lp_vendor(const void* a, const void* b, void* c, int ab_dty
 
 int mcke_gemm_mfma_default_tile(int64_t m, int64_t n, int64_t k, mcke_gemm_tile* out) {
   if (!out) return invalid("gemm_mfma_default_tile: null out");
-  // The tile whose launch is the shortest (tile_us), ties to the larger one; the 64 x 64
-  // tile counts as the better of its own and the 32 x 64 one that it may run.  Shapes that
-  // are not whole tiles cost the two large tiles 3% more (the EDGE form's row and column
-  // checks: 1000 x 4096 x 1024 69.8 us against 68.0 for 1024 rows at 128 x 128).
+  // The tile whose launch is the shortest (tile_us, scaled to K up to 256 and with the tiles'
+  // fixed cost), ties to the larger one; the 64 x 64 tile counts as the better of its own and
+  // the 32 x 64 one that it may run where N and K are 64 or more.  Shapes that are not whole tiles cost the
+  // two large tiles 3% more (the EDGE form's row and column checks: 1000 x 4096 x 1024 69.8 us
+  // against 68.0 for 1024 rows at 128 x 128).
   static const mcke_gemm_tile cands[] = {
       {256, 256, 32, 16, 16}, {128, 128, 32, 8, 8}, {64, 64, 32, 4, 4}, {32, 32, 32, 2, 2}};
   const int64_t cus = device_cu_count();
+  auto launch_us = [&](int bm, int bn) {
+    const double us = tile_us(bm, bn, m, n, cus);
+    if (k > 256) return us;
+    return us * static_cast<double>(k) / 4096.0 + tile_fixed_us(bm, bn, m, n, cus);
+  };
   double best = 0.0;
   for (const mcke_gemm_tile& c : cands) {
-    double us = tile_us(c.bm, c.bn, m, n, cus);
-    if (c.bm == 64) us = std::min(us, tile_us(32, 64, m, n, cus));
+    double us = launch_us(c.bm, c.bn);
+    if (c.bm == 64 && n >= 64 && k >= 64) us = std::min(us, launch_us(32, 64));
     if (c.bm >= 128 && (m % c.bm != 0 || n % c.bn != 0 || k % 32 != 0)) us *= 1.03;
     if (c.bm == 256 || us < best) {
       best = us;

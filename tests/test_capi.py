@@ -181,6 +181,10 @@ def test_default_mfma_tile(mcke):
     assert mcke.gemm_mfma_default_tile(1024, 1024, 1024).astuple() == (64, 64, 32, 4, 4)
     # 512^3: 64 tiles of 64 fill a quarter round; 256 tiles of 32 fill one.
     assert mcke.gemm_mfma_default_tile(512, 512, 512).astuple() == (32, 32, 32, 2, 2)
+    # Short K: a tile's fixed cost counts, so many small tiles do not win.
+    for mnk in ((576, 3904, 1), (576, 3904, 48), (499, 4388, 32), (3458, 616, 96),
+                (4605, 344, 100), (4480, 800, 40), (4614, 6836, 16)):
+        assert mcke.gemm_mfma_default_tile(*mnk).astuple() == (64, 64, 32, 4, 4), mnk
     assert mcke.gemm_mfma_default_tile(256, 256, 256).astuple() == (32, 32, 32, 2, 2)
     assert mcke.gemm_mfma_default_tile(1, 1, 1).astuple() == (32, 32, 32, 2, 2)
 

@@ -52,14 +52,9 @@ def test_gemm_f32_tile_edges(gpu, orc, t):
             del da, db
 
 
-# 64 x 64 launches that run 128 x 64 tiles (1000 x 4096: four 64 x 64 tiles per CU) and
-# 32 x 64 tiles (1531 x 1021: 1.5 per CU), whole and not.
-@pytest.mark.parametrize("shape", [(1024, 4096, 64), (1000, 4093, 70), (901, 4096, 33),
-                                   (1536, 1024, 96), (1531, 1021, 70), (1505, 1089, 32)],
-                         ids=lambda s: "x".join(map(str, s)))
-def test_64_tile_launch_picks(gpu, orc, shape):
+def _check_plain_and_fused(gpu, orc, shape, tile):
     M, N, K = shape
-    V, tile = gpu.GemmVariant.kMfmaF32, _tile(gpu, 64)
+    V = gpu.GemmVariant.kMfmaF32
     a = orc.fill_random(M * K, 61 + K).reshape(M, K)
     b = orc.fill_random(K * N, 62 + N).reshape(K, N)
     c = orc.fill_random(M * N, 63 + M).reshape(M, N)
@@ -90,6 +85,31 @@ def test_64_tile_launch_picks(gpu, orc, shape):
         del da, db
 
 
+# 64 x 64 launches that run 128 x 64 tiles (1000 x 4096: four 64 x 64 tiles per CU) and
+# 32 x 64 tiles (1531 x 1021: 1.5 per CU), whole and not.
+@pytest.mark.parametrize("shape", [(1024, 4096, 64), (1000, 4093, 70), (901, 4096, 33),
+                                   (1536, 1024, 96), (1531, 1021, 70), (1505, 1089, 32)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_64_tile_launch_picks(gpu, orc, shape):
+    _check_plain_and_fused(gpu, orc, shape, _tile(gpu, 64))
+
+
+# Launches of the small tiles that run the tile's own EDGE kernel: one 64 x 64 tile per CU,
+# where 32 x 64 ones tie, and more 32 x 32 tiles than the few-tiles kernel takes.
+OWN_EDGE = ([(64, (1000, 1023, k)) for k in (33, 64, 95, 161, 333)] +
+            [(32, (500, 515, k)) for k in (64, 65, 95, 161, 319)])
+# K of 32 to 63: with 16-byte operands (and at 32 x 32) the staged kernel, whole tiles of 64
+# their own where 128 x 64 ones (960 rows) would not be whole.
+SHORT_K = [(64, (996, 1020, 32)), (64, (996, 1020, 40)), (64, (960, 4096, 32)),
+           (128, (260, 388, 32)), (256, (260, 516, 60)), (32, (500, 516, 60)), (32, (500, 515, 33))]
+
+
+@pytest.mark.parametrize("t,shape", OWN_EDGE + SHORT_K,
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_tile_own_kernels(gpu, orc, t, shape):
+    _check_plain_and_fused(gpu, orc, shape, _tile(gpu, t))
+
+
 @pytest.mark.parametrize("t", TILES)
 @pytest.mark.parametrize("act", [0, 1, 2, 3])
 def test_fused_tile_edges_match_the_pair(gpu, orc, t, act):
@@ -113,11 +133,15 @@ def test_fused_tile_edges_match_the_pair(gpu, orc, t, act):
         del da, db, dbias
 
 
-@pytest.mark.parametrize("t", TILES)
-def test_gemm_remainder_keeps_special_values_apart(gpu, orc, t):
+@pytest.mark.parametrize("t,shape", [(t, (t + 1, t + 5, 45)) for t in TILES] +
+                         [(64, (1000, 1023, 45)), (32, (500, 515, 77))],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_gemm_remainder_keeps_special_values_apart(gpu, orc, t, shape):
     """K % 32 != 0 pads both operands with zeros: infinities and NaN in the last columns of
-    A, the last rows of B, and past the operands' ends reach their own outputs only."""
-    M, N, K = t + 1, t + 5, 45
+    A, the last rows of B, and past the operands' ends reach their own outputs only.  (At t +
+    1 x t + 5 the 64 x 64 launch runs 32 x 64 tiles and the 32 x 32 one the few-tiles kernel;
+    the last two shapes run the tile's own EDGE kernel.)"""
+    M, N, K = shape
     a = orc.fill_random(M * K, 31).reshape(M, K)
     b = orc.fill_random(K * N, 32).reshape(K, N)
     a[M - 1, 3], a[0, K - 1] = np.nan, np.inf

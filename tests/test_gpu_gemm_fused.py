@@ -90,6 +90,19 @@ def test_whole_tiles_match_the_pair_and_the_oracle(gpu, orc, ti, act):
         _check_oracle(orc, fused, _oracle(orc, a, b, bias, M, N, K, alpha, act), K)
 
 
+# _whole_shape of the two small tiles runs the 32 x 64 tile and the few-tiles kernel; these
+# shapes run the 64 x 64 and 32 x 32 tiles' own kernels.
+@pytest.mark.parametrize("k", [32, 64, 96, 160, 224])
+@pytest.mark.parametrize("ti,M,N", [(4, 1024, 1024), (5, 512, 544)])
+def test_small_tiles_own_kernels_match_the_pair_and_the_oracle(gpu, orc, ti, M, N, k):
+    t = gpu.MFMA_TILES[ti]
+    a, b, bias = _inputs(orc, M, N, k, ti)
+    for act in ACTS:
+        fused, pair = _run(gpu, a, b, bias, M, N, k, -0.75, act, t)
+        assert _nan_aware_bits_equal(fused, pair), (t.astuple(), act)
+    _check_oracle(orc, fused, _oracle(orc, a, b, bias, M, N, k, -0.75, ACTS[-1]), k)
+
+
 @pytest.mark.parametrize("ti", range(6), ids=lambda i: f"tile{i}")
 @pytest.mark.parametrize("shape", [(129, 65, 257), (33, 63, 1), (1, 64, 128), (253, 253, 253)],
                          ids=lambda s: "x".join(map(str, s)))

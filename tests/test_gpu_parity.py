@@ -451,10 +451,10 @@ def test_gemm_512_baseline_config(gpu, orc):
 
 
 def test_mfma_kernel_attrs_report_the_whole_tile_kernel(gpu):
-    """gemm_kernel_attrs (kernels.hpp:293-302) describes the kernel that whole-tile
-    shapes run: the 64x64, 128x128 and 256x256 tiles' direct-to-LDS kernels run
-    one wave group of four waves (256 lanes), the 32x32 tile four one-wave groups
-    (256 lanes)."""
+    """gemm_kernel_attrs (kernels.hpp:293-302) describes the tile's own direct-to-LDS
+    kernel: the 64x64, 128x128 and 256x256 ones run one wave group of four waves (256
+    lanes), the 32x32 one four one-wave groups (256 lanes).  (A launch of a small tile may
+    run another kernel of its size class.)"""
     T = gpu.GemmTile
     for tile, threads in ((T(32, 32, 32, 2, 2), 256), (T(64, 64, 32, 4, 4), 256),
                           (T(128, 128, 32, 8, 8), 256), (T(256, 256, 32, 16, 16), 256)):
@@ -464,7 +464,13 @@ def test_mfma_kernel_attrs_report_the_whole_tile_kernel(gpu):
         assert at.max_blocks_per_sm_api >= 1 and at.local_bytes == 0, tile.astuple()
 
 
+# The 64x64 and 32x32 tiles' own kernels run where 64x64 tiles are one to a CU (1024x1024),
+# and where the product is more 32x32 tiles than the few-tiles kernel takes (512x544).  The
+# small shapes of these tiles run the 32x64 tile (two wave groups over K) and the few-tiles
+# kernel.
 _DMA_STEP_CASES = (
+    [((64, 64, 32, 4, 4), (1024, 1024, k)) for k in (32, 64, 96, 160, 224)] +
+    [((32, 32, 32, 2, 2), (512, 544, k)) for k in (32, 64, 96, 160, 224)] +
     [((64, 64, 32, 4, 4), mnk) for mnk in
      [(128, 128, 32), (128, 128, 96), (192, 64, 160), (64, 128, 224), (64, 64, 64)]] +
     [((32, 32, 32, 2, 2), mnk) for mnk in [(128, 128, 32), (128, 128, 96), (64, 96, 160)]] +
@@ -503,10 +509,10 @@ def test_gemm_dma_ring_step_counts(gpu, orc, tile, mnk):
 @pytest.mark.parametrize("tile", [(64, 64, 32, 4, 4), (32, 32, 32, 2, 2)])
 @pytest.mark.parametrize("n", [32, 64, 192, 512, 1024, 100, 257])
 def test_gemm_wave_group_tiles(gpu, orc, tile, n):
-    """The small tiles: 64x64 (one wave group, 4-stage mid-step ring) and 32x32,
-    which folds its four wave groups' shares of K in a fixed order (whole tiles on
-    the direct-to-LDS kernel; n = 100 and 257 on the staged kernel, whose 32x32
-    tile also runs four groups): the full reference (reference.hpp:199-211) at the
+    """The small tiles' size classes: 64x64 (whole tiles of 64x64 at n = 1024, 32x64
+    tiles below) and 32x32 (the few-tiles kernel, whose eight waves split K, up to n =
+    257 and past that at n = 512 and 1024 the tile's four wave groups, folded in a fixed
+    order): the full reference (reference.hpp:199-211) at the
     K-scaled tolerance, the same bits on a second launch, and beta = 0 never
     reading a NaN-poisoned C."""
     a = orc.fill_random(n * n, 0x6E33A + n)
