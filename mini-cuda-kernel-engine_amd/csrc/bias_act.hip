@@ -15,9 +15,10 @@
 //     wave's life is short (its row and strip come from a multiply-shift
 //     division, no loop), and the hardware streams workgroups through the CUs in
 //     address order;
-//   * launches with a capped grid (max_row_blocks, the reference's starvation
-//     lever) and tensors beyond the flat grids' 32-bit limits: a 2-D grid of column strips x row blocks that walks rows with a
-//     stride of gridDim.y, four per iteration (4 / VW rows per workgroup at once);
+//   * launches with a capped grid (max_row_blocks, the reference's starvation lever) and
+//     tensors beyond the flat grids' 32-bit limits: a 2-D grid of column strips x row
+//     blocks that walks rows with a stride of gridDim.y, four per iteration (4 / VW rows
+//     per workgroup at once);
 //   * small launches (at most two rounds of resident workgroups at one row each):
 //     256-lane workgroups that each own kChunkRows adjacent rows of their column
 //     strip and issue all their loads before any store, so the launch is one
@@ -36,8 +37,8 @@ namespace {
 
 constexpr int kThreads = 256;
 // Workgroups of the row kernel move kRowBytes of a row: one wave at VW = 4, 128
-// lanes at VW = 2, 256 at VW = 1, each workgroup over 4 / VW rows at once.  The flat activation kernel
-// runs one-wave workgroups (kRowLanes).  On gfx950 one-wave workgroups each
+// lanes at VW = 2, 256 at VW = 1, each workgroup over 4 / VW rows at once.  The flat
+// activation kernel runs one-wave workgroups (kRowLanes).  On gfx950 one-wave workgroups each
 // moving one 16-byte vector per lane streamed a 2 x 256 MiB copy 3% faster than
 // 256-lane workgroups of the same shape (80.0 vs 82.5 us); workgroups moving less
 // than 1 KiB a row are slower again (GELU_tanh at 16384 x 4096 with one-wave

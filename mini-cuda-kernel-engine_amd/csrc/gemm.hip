@@ -740,9 +740,9 @@ int mcke_gemm_mfma_default_tile(int64_t m, int64_t n, int64_t k, mcke_gemm_tile*
   if (!out) return invalid("gemm_mfma_default_tile: null out");
   // The tile whose launch is the shortest (tile_us, scaled to K up to 256 and with the tiles'
   // fixed cost), ties to the larger one; the 64 x 64 tile counts as the better of its own and
-  // the 32 x 64 one that it may run where N and K are 64 or more.  Shapes that are not whole tiles cost the
-  // two large tiles 3% more (the EDGE form's row and column checks: 1000 x 4096 x 1024 69.8 us
-  // against 68.0 for 1024 rows at 128 x 128).
+  // the 32 x 64 one that it may run where N and K are 64 or more.  Shapes that are not whole
+  // tiles cost the two large tiles 3% more (the EDGE form's row and column checks: 1000 x 4096
+  // x 1024 69.8 us against 68.0 for 1024 rows at 128 x 128).
   static const mcke_gemm_tile cands[] = {
       {256, 256, 32, 16, 16}, {128, 128, 32, 8, 8}, {64, 64, 32, 4, 4}, {32, 32, 32, 2, 2}};
   const int64_t cus = device_cu_count();

@@ -71,7 +71,7 @@ int launch_split_as(const LpArgs& x) {
   constexpr int TM = 16 * MT, TN = 16 * NW;
   const int64_t tiles = tile_count(x.m, x.n, TM, TN);
   if (int rc = check_grid(tiles, WV * kWave)) return rc;
-  gemm_lp_split_kernel<T, OutT, MT, NW, WV, 1>
+  gemm_lp_split_kernel<T, OutT, MT, NW, WV>
       <<<static_cast<unsigned>(tiles), WV * kWave, 0, x.s>>>(
           x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
           tiles_along(x.m, TM), tiles_along(x.n, TN));
@@ -81,10 +81,10 @@ int launch_split_as(const LpArgs& x) {
 
 // The split-K kernel by shape.  Few rows over up to 8192 columns: 32 columns a workgroup
 // and 8 waves, for as many workgroups as there are (16 x 4096 x 4096: 16 x 32 11.9 us,
-// 32 x 64 16.1, 64 x 64 18.9; 16 x 16384 x 4096: 38.5, 27.1, 29.0).  Else 32 x 64 up to
-// four tiles per CU (64 x 4096 x 4096: 16.7 us against 21.3 for 64 x 64; 1628 x 800 x 1109:
-// 18.2 against 20.3), 64 x 64 past that (1531 x 4096 x 1024: 34.0 against 40.3;
-// 4032 x 843 x 2744: 70.2 against 86.1).  Widths of 32 .. 63 take 32 columns.
+// 32 x 64 14.8, 64 x 64 16.4; 16 x 16384 x 4096: 38.6, 25.8, 26.8).  Else 32 x 64 up to
+// four tiles per CU (64 x 4096 x 4096: 15.6 us against 21.3 for 64 x 64; 1628 x 800 x 1109:
+// 14.9 against 17.4), 64 x 64 past that (1531 x 4096 x 1024: 28.2 against 33.3;
+// 4032 x 843 x 2744: 62.7 against 83.8).  Widths of 32 .. 63 take 32 columns.
 template <typename T, typename OutT>
 int launch_split(const LpArgs& x) {
   if (x.n < 64 || (x.m <= 32 && x.n <= 8192))
@@ -110,10 +110,10 @@ int launch_staged(const LpArgs& x, bool vec) {
 
 // Short K over many tiles: the product is its C store, and the register-staged kernel's four
 // waves share a tile's one stage where the split-K kernel has one wave work and three add
-// zeros.  16-byte operands up to 63 of K (fp16 to fp32, 2460 x 1608 x 40: 7.6 us at 64 x 64
-// against 10.7 for split K; up to 1024 tiles they tie, 1101 x 1104 x 40 4.98 against 4.6),
-// others up to 7, as their loads are element by element (2460 x 1607 x 7: 10.2 against 11.1;
-// x 16: 11.8 against 9.9).  128 x 128 tiles where they fill two rounds of CUs or more to 80%
+// zeros.  16-byte operands up to 63 of K (fp16 to fp16, 2460 x 1608 x 40: 6.7 us at 64 x 64
+// against 9.9 for split K; up to 1024 tiles they tie, fp32 C, 853 x 1880 x 64 5.5 against 5.4),
+// others up to 7, as their loads are element by element (fp32 C, 2293 x 1737 x 7: 10.3 against
+// 12.8; x 15: 11.6 against 11.7).  128 x 128 tiles where they fill two rounds of CUs or more to 80%
 // (2166 x 3544 x 40: 10.9 us against 12.1 at 64 x 64; 2460 x 1608, 260 tiles: 10.3 against 7.6).
 bool short_k(const LpArgs& x, bool vec) {
   return x.k < (vec ? 64 : 8) && tile_count(x.m, x.n, 32, 64) > 1024;
@@ -122,7 +122,8 @@ bool short_k(const LpArgs& x, bool vec) {
 template <typename T, typename OutT>
 int launch_short_k(const LpArgs& x, bool vec) {
   const int64_t tiles = tile_count(x.m, x.n, 128, 128), rounds = (tiles + 255) / 256;
-  if (rounds >= 2 && 10 * tiles >= 8 * 256 * rounds) return launch_staged<T, OutT, 128, 128>(x, vec);
+  if (rounds >= 2 && 10 * tiles >= 8 * 256 * rounds)
+    return launch_staged<T, OutT, 128, 128>(x, vec);
   return launch_staged<T, OutT, 64, 64>(x, vec);
 }
 
@@ -131,9 +132,10 @@ template <typename T, typename OutT, int BM, int BN>
 int launch_whole(const LpArgs& x) {
   const int64_t tiles = tile_count(x.m, x.n, BM, BN);
   if (int rc = check_grid(tiles, kMfmaThreads)) return rc;
-  gemm_lp_kernel<T, OutT, BM, BN, false, true><<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
-      x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
-      tiles_along(x.m, BM), tiles_along(x.n, BN));
+  gemm_lp_kernel<T, OutT, BM, BN, false, true>
+      <<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
+          x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
+          tiles_along(x.m, BM), tiles_along(x.n, BN));
   MCKE_LAUNCH_CHECK("gemm_lp_kernel");
   return ok();
 }
@@ -167,19 +169,19 @@ template <typename T, typename OutT, int BM, int BN>
 struct LpTile {
   // Whole tiles run the requested tile's direct-to-LDS kernel (tiles of 128 and more).
   // Other shapes run its EDGE form, at 128 x 128 from 208 such tiles on, or from 80 on where
-  // K is long enough to pay for a tile alone on its CU, and at 256 x 256
-  // where they nearly fill the CUs (fp16 to fp32: 2757 x 432 x 6080, 88 tiles of 128,
-  // 49.9 us against 54.9 for split K; 1628 x 800 x 1110, 91 tiles, 17.2 against 18.2;
-  // 300 x 520 x 1032, 15 tiles, 15.4 against 6; 4524 x 344 x 96, 108 tiles, 7.5 against 5.4,
-  // to fp16 5.6 against 5.1; 4095 x 4094 x 4090, 256 tiles of 256,
-  // 130 us against 205 at 128).  Odd extents run the register-staged kernel's WHOLE form
-  // where its 128 x 128 tiles fill most of the CUs (a tile alone on its CU takes 1.3 us per
-  // 64 of K, so fewer lose to split K: 1531 x 1021 x 2053, 96 tiles, 44.3 us against 31.5;
-  // 1700 x 1701 x 1024, 196 tiles, 23.9 against 21.6; 4032 x 843 x 2744, 224 tiles, 54.0
-  // against 68.7; 1901 x 2001 x 511, 240 tiles, 20.3 against 30.4; 3001 x 2501 x 901, 480
-  // tiles, 32.8 against 57.1), at 256 x 256 from 192 such tiles on (4095^3 191 us against
-  // 229 at 128 and 395 for split K; 3500 x 3501 x 2001, 196 tiles, 98 against 102).  What is
-  // left takes the split-K kernel, as every 64 x 64 launch does.
+  // K is long enough to pay for a tile alone on its CU, and at 256 x 256 where they nearly
+  // fill the CUs (fp16 to fp32: 2757 x 432 x 6080, 88 tiles of 128, 49.8 us against 56.9 for
+  // split K; 1628 x 800 x 1110, 91 tiles, 15.9 against 15.2; 300 x 520 x 1032, 15 tiles, 14.4
+  // against 7.6; 4524 x 344 x 96, 108 tiles, 7.5 against 5.8, to fp16 5.9 against 5.5;
+  // 4095 x 4094 x 4090, 256 tiles of 256, 126 us against 206 at 128).  Odd extents run the
+  // register-staged kernel's WHOLE form where its 128 x 128 tiles fill most of the CUs (a tile
+  // alone on its CU takes 1.3 us per 64 of K, so fewer lose to split K: 1531 x 1021 x 2053, 96
+  // tiles, 44.4 us against 29.9; 1700 x 1701 x 1024, 196 tiles, 24.0 against 20.8;
+  // 4032 x 843 x 2744, 224 tiles, 54.5 against 63.9; 1901 x 2001 x 511, 240 tiles, 20.4 against
+  // 22.1; 3001 x 2501 x 901, 480 tiles, 33.1 against 50.0), at 256 x 256 from 192 such tiles on
+  // (4095^3 199 us against 229 at 128 and 406 for split K; 3500 x 3501 x 2001, 196 tiles, 99
+  // against 105).  What is left takes the split-K kernel, as 64 x 64 launches do, but for
+  // short K over many tiles (short_k).
   static int launch(const LpArgs& x, bool vec) {
     if constexpr (BN >= 128) {
       if (vec && x.m % BM == 0 && x.n % BN == 0 && x.k % 64 == 0 && x.k > 0 &&
@@ -216,7 +218,7 @@ struct LpTile {
     if constexpr (BN >= 128)
       return reinterpret_cast<LpKernel>(&gemm_lp_dma16_kernel<T, OutT, BM, BN, false>);
     else
-      return reinterpret_cast<LpKernel>(&gemm_lp_split_kernel<T, OutT, 4, 4, 4, 1>);
+      return reinterpret_cast<LpKernel>(&gemm_lp_split_kernel<T, OutT, 4, 4, 4>);
   }
 };
 
@@ -346,7 +348,8 @@ int mcke_gemm_lp_default_tile(int64_t m, int64_t n, int64_t k, mcke_gemm_tile* o
   // The largest tile that still fills most of a 256-CU part.  Measured on MI355X: 256 x 256
   // wins at 4096^3 (256 tiles) and at 3072 x 4096 x 1024 (192 tiles, bf16: 32.1 us against
   // 33.6), 128 x 128 at 2048^3 (256 tiles: 23.2 us against 37.2 for 64 x 64) and down to
-  // 1628 x 800 (91 tiles), 64 x 64 at 1024^3 (64 tiles of 128: 12.4 us against 8.8).
+  // 80 tiles (a launch of fewer than 208 that are not whole still splits K where K is short or
+  // odd), 64 x 64 at 1024^3 (64 tiles of 128: 12.4 us against 8.8).
   auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
   if (tiles(256) >= 192) *out = mcke_gemm_tile{256, 256, kLpBK, 16, 16};
   else if (tiles(128) >= 80) *out = mcke_gemm_tile{128, 128, kLpBK, 8, 8};

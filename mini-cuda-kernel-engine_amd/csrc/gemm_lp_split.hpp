@@ -6,10 +6,10 @@
 // tile this small a 2 x 2 wave grid reads each operand from LDS twice (256 bytes per
 // cycle at 64 x 64 for 16x16x32 MFMAs, twice what LDS delivers) and meets at a barrier
 // for a few MFMAs' worth of work.  Here
-//   * every wave computes the whole 16 MT x 16 NW tile over its own K chunks (32 H deep,
-//     dealt to the WV waves in turn), so a fragment is read from LDS once, and the loop
-//     has no barrier: a wave loads a chunk into registers, writes it to an LDS slot of its
-//     own while the next chunk's loads are in flight, and reads the fragments back;
+//   * every wave computes the whole 16 MT x 16 NW tile over its own K chunks (32 deep, dealt
+//     to the WV waves in turn), so a fragment is read from LDS once, and the loop has no
+//     barrier: a wave loads a chunk into registers, writes it to an LDS slot of its own while
+//     the next chunk's loads are in flight, and reads the fragments back;
 //   * loads are 16 bytes per lane at 2-byte alignment, so odd widths and unaligned
 //     operands take the same path (the register-staged kernel loads them 2 bytes at a
 //     time);
@@ -17,18 +17,21 @@
 //   * the waves' sums are folded through LDS in a fixed order at the end.
 //
 // Measured on MI355X, fp16 to fp32, four sets of operands in turn (us; the
-// register-staged kernel, 64 x 64 tile, then this):
-//   16 x 4096 x 4096  46.6  11.8 (16 x 32, 8 waves)   1024^3           14.9   8.4 (64 x 64)
-//   64 x 4096 x 4096  47.3  17.9 (64 x 32, 8 waves)   317 x 304 x 960  13.4   6.1 (64 x 32)
-//   9 x 5184 x 1523   58.7   8.2 (16 x 64, 8 waves)   1628 x 800 x 1109  77.5  20.4 (64 x 64)
-//   36 x 7379 x 8064   409  42.3 (64 x 32)            4032 x 843 x 2744   254  70.7 (64 x 64)
-// Direct-to-LDS loads in the same scheme are within 6% either way (16 x 4096 x 4096 12.4,
-// 1024^3 7.9) and need 4-byte alignment.
+// register-staged kernel, 64 x 64 tile, then this one in the configuration that the
+// launcher picks):
+//   16 x 32, 8 waves:  16 x 4096 x 4096  46.5  12.1    9 x 5184 x 1523     58.9   5.7
+//   32 x 32, 8 waves:  32 x 4096 x 4096  47.1  13.8
+//   32 x 64, 4 waves:  64 x 4096 x 4096  47.5  15.7    1024^3              15.4   8.6
+//                      36 x 7379 x 8064   411  45.9    317 x 304 x 960     12.5   5.5
+//                      1628 x 800 x 1109 77.4  15.6    1531 x 1021 x 2053   123  29.4
+//   64 x 64, 4 waves:  1700 x 1501 x 1024  85.8  20.4
+// Direct-to-LDS loads in the same scheme are within 6% either way (16 x 4096 x 4096 12.4
+// against 11.8 in one sweep, 1024^3 7.9 against 8.4) and need 4-byte alignment.
 //
-// LDS slot of a wave, per chunk: H KB per 16 rows of A, rows of 64 H bytes with 16-byte
-// quad q of row r at q ^ aswz(r); per 32 k, NW KB of B: k = 8 g + 4 t + j sits at
-// position s = 16 t + 4 g + j (a transposed read takes one t), 32-byte column block b of
-// a position at b ^ bswz(s).  Both put what a half-wave reads on distinct banks.
+// LDS slot of a wave, per chunk: 1 KB per 16 rows of A, rows of 64 bytes with 16-byte quad q
+// of row r at q ^ aswz(r); NW KB of B: k = 8 g + 4 t + j sits at position
+// s = 16 t + 4 g + j (a transposed read takes one t), 32-byte column block b of a position
+// at b ^ bswz(s).  Both put what a half-wave reads on distinct banks.
 #pragma once
 
 #include "gemm_lp.hpp"
@@ -37,11 +40,11 @@ namespace mcke_amd {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-template <int MT, int NW, int WV, int H>
+template <int MT, int NW, int WV>
 struct LpSplitShape {
   static constexpr int TM = 16 * MT, TN = 16 * NW;
-  static constexpr int KC = 32 * H;                       // K per chunk
-  static constexpr int NA = MT * H, NB = NW * H;          // 1 KB loads per chunk
+  static constexpr int KC = 32;                           // K per chunk
+  static constexpr int NA = MT, NB = NW;                  // 1 KB loads per chunk
   static constexpr int L = NA + NB;
   static constexpr int kSlot = L * 1024;
   static constexpr int kThreads = WV * 64;
@@ -52,18 +55,19 @@ struct LpSplitShape {
   static constexpr int kFold = kOut * 4 * WV <= kSlots ? WV : WV / 2;
   static constexpr int kLds = kSlots > kFold * kOut * 4 ? kSlots : kFold * kOut * 4;
   static_assert(kLds <= 64 * 1024, "two workgroups or more per CU");
-  static constexpr int kARow = 64 * H, kBRow = 32 * NW;
-  static __host__ __device__ constexpr int aswz(int r) { return H == 2 ? (r >> 1) & 7 : (r >> 2) & 3; }
+  static constexpr int kARow = 64, kBRow = 32 * NW;
+  static_assert(NW == 2 || NW == 4, "column blocks are swizzled in twos or fours");
+  static __host__ __device__ constexpr int aswz(int r) { return (r >> 2) & 3; }
   static __host__ __device__ constexpr int bswz(int s) {
-    return NW == 1 ? 0 : NW == 2 ? (s >> 2) & 1 : (s >> 1) & 3;
+    return NW == 2 ? (s >> 2) & 1 : (s >> 1) & 3;
   }
 };
 
-template <typename T, typename OutT, int MT, int NW, int WV, int H>
+template <typename T, typename OutT, int MT, int NW, int WV>
 __global__ __launch_bounds__(WV * 64) void gemm_lp_split_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, OutT* __restrict__ C, int M,
     int N, int K, float alpha, float beta, int tiles_m, int tiles_n) {
-  using S = LpSplitShape<MT, NW, WV, H>;
+  using S = LpSplitShape<MT, NW, WV>;
   constexpr int L = S::L;
   __shared__ __attribute__((aligned(1024))) char smem[S::kLds];
 
@@ -81,24 +85,21 @@ __global__ __launch_bounds__(WV * 64) void gemm_lp_split_kernel(
   // column starts at N - TN and stores only the columns of its own.
   // a_k and b_k: the first k of the lane's eight in A, and its k in B.
   uint32_t a_src[S::NA], b_src[S::NB];
-  int a_k[S::NA], b_k[S::NB];
+  int b_k[S::NB];
+  const int a_row = lane / 4, a_quad = (lane % 4) ^ S::aswz(a_row), a_k = 8 * a_quad;
 #pragma unroll
   for (int i = 0; i < S::NA; ++i) {
-    const int at = (i % H) * 1024 + 16 * lane;
-    const int r = at / S::kARow, row_t = 16 * (i / H) + r;
+    const int row_t = 16 * i + a_row;
     const int row = row_t > M - 1 - m0 ? M - 1 - m0 : row_t;
-    const int q = ((at % S::kARow) / 16) ^ S::aswz(r);
-    a_k[i] = 8 * q;
-    a_src[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) * 2u + 16u * q;
+    a_src[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) * 2u + 16u * a_quad;
   }
 #pragma unroll
   for (int u = 0; u < S::NB; ++u) {
-    const int at = (u % NW) * 1024 + 16 * lane;
+    const int at = u * 1024 + 16 * lane;
     const int s = at / S::kBRow;
     const int b = ((at % S::kBRow) / 32) ^ S::bswz(s);
-    const int k = 32 * (u / NW) + 8 * ((s / 4) % 4) + 4 * (s / 16) + s % 4;
-    b_k[u] = k;
-    b_src[u] = (static_cast<uint32_t>(k) * static_cast<uint32_t>(N) + 16u * b) * 2u +
+    b_k[u] = 8 * ((s / 4) % 4) + 4 * (s / 16) + s % 4;
+    b_src[u] = (static_cast<uint32_t>(b_k[u]) * static_cast<uint32_t>(N) + 16u * b) * 2u +
                static_cast<uint32_t>(at % 32);
   }
   const char* a_base = reinterpret_cast<const char*>(A + static_cast<int64_t>(m0) * K);
@@ -106,9 +107,8 @@ __global__ __launch_bounds__(WV * 64) void gemm_lp_split_kernel(
   char* slot = smem + wave * S::kSlot;
 
   // Fragment addresses within a slot.
-  uint32_t a_off[H], b_off[NW];
-#pragma unroll
-  for (int h = 0; h < H; ++h) a_off[h] = c * S::kARow + 16 * ((4 * h + g) ^ S::aswz(c));
+  const uint32_t a_off = c * S::kARow + 16 * (g ^ S::aswz(c));
+  uint32_t b_off[NW];
 #pragma unroll
   for (int b = 0; b < NW; ++b) {
     const int s = g * 4 + c / 4;                        // read t adds 16 positions
@@ -124,30 +124,26 @@ __global__ __launch_bounds__(WV * 64) void gemm_lp_split_kernel(
   const int chunks = K / S::KC;
   const int n_it = chunks > wave ? (chunks - wave + WV - 1) / WV : 0;
   auto compute = [&]() {
+    u32x4 av[MT];
+    u32x2 bv[NW][2];
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
-      u32x4 av[MT];
-      u32x2 bv[NW][2];
+    for (int m = 0; m < MT; ++m) av[m] = *reinterpret_cast<const u32x4*>(slot + m * 1024 + a_off);
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        av[m] = *reinterpret_cast<const u32x4*>(slot + m * (H * 1024) + a_off[h]);
+    for (int b = 0; b < NW; ++b)
 #pragma unroll
-      for (int b = 0; b < NW; ++b)
+      for (int t = 0; t < 2; ++t)
+        bv[b][t] = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                       (__attribute__((address_space(3))) s16x4*)(
+                           slot + t * (16 * S::kBRow) + b_off[b])));
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-          bv[b][t] = __builtin_bit_cast(
-              u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                         (__attribute__((address_space(3))) s16x4*)(
-                             slot + h * (NW * 1024) + t * (16 * S::kBRow) + b_off[b])));
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int bb = 0; bb < NW; ++bb) {
-          const int b = mfma_snake_col(m, bb, NW);
-          acc[m][b] = LpMfma16<T>::run(
-              av[m], u32x4{bv[b][0][0], bv[b][0][1], bv[b][1][0], bv[b][1][1]}, acc[m][b]);
-        }
-    }
+      for (int bb = 0; bb < NW; ++bb) {
+        const int b = mfma_snake_col(m, bb, NW);
+        acc[m][b] = LpMfma16<T>::run(
+            av[m], u32x4{bv[b][0][0], bv[b][0][1], bv[b][1][0], bv[b][1][1]}, acc[m][b]);
+      }
   };
 
   auto load = [&](int it, u32x4 (&v)[L]) {
@@ -184,16 +180,15 @@ __global__ __launch_bounds__(WV * 64) void gemm_lp_split_kernel(
 #pragma unroll
     for (int i = 0; i < S::NA; ++i) {
       w[i] = u32x4{0u, 0u, 0u, 0u};
-      if (a_k[i] + 8 <= rem) {
+      if (a_k + 8 <= rem) {
         w[i] = *reinterpret_cast<const u32x4_a2*>(ap + a_src[i]);
-      } else if (a_k[i] < rem) {
+      } else if (a_k < rem) {
         if (K >= 8) {
           const u32x4 last8 = *reinterpret_cast<const u32x4_a2*>(ap + a_src[i] - 2 * past);
           w[i] =
               __builtin_bit_cast(u32x4, __builtin_bit_cast(unsigned __int128, last8) >> (16 * past));
         } else {
-          w[i] =
-              lp_load8<false>(reinterpret_cast<const uint16_t*>(ap + a_src[i]), a_k[i], rem, true);
+          w[i] = lp_load8<false>(reinterpret_cast<const uint16_t*>(ap + a_src[i]), a_k, rem, true);
         }
       }
     }
