@@ -7,8 +7,8 @@
 //   * GemmVariant is append-only and gains kMfmaF32 (= 8), whose tiles are
 //     (256,256,32,16,16), (256,256,16,16,16), (128,128,32,8,8), (128,128,16,8,8),
 //     (64,64,32,4,4) and (32,32,32,2,2): 256 lanes in the (bm/tm) x (bn/tn)
-//     descriptor (the whole-tile kernels of the two smallest tiles split each
-//     K stage over wave groups; the descriptor stays the tile's identity);
+//     descriptor (a launch of the two smallest may run other tiles of their size
+//     class, up to 512 lanes; the descriptor stays the tile's identity);
 //   * occupancy is limited per SIMD by the 512-entry unified VGPR file (arch +
 //     accumulation registers, allocated in granules of 8) and 8 waves, per CU by
 //     160 KiB of LDS, the 2048-lane cap and the workgroup cap.

@@ -171,8 +171,11 @@ int mcke_launch_row_softmax_f32(const float* x, float* y, int64_t rows, int64_t 
  * C = alpha*A[m,k]B[k,n] + beta*C, row-major.  C is not read when beta == 0.
  * m == 0 or n == 0 is a no-op; k == 0 gives C = beta*C.  a == c or b == c,
  * negative or > INT32_MAX extents, and (variant, tile) pairs that are not
- * compiled are INVALID_ARGUMENT (no fallback tile).  kMfmaF32's 32 x 32 and 64 x 64 tiles name
- * a size class: a launch runs the class's kernel whose tiles fill the GPU best. */
+ * compiled are INVALID_ARGUMENT (no fallback tile).  A kMfmaF32 tile names a size
+ * class: by shape and alignment a launch runs the tile's direct-to-LDS kernel, its
+ * form for shapes that are not whole tiles or its register-staged kernel; a 64 x 64
+ * one may run 128 x 64 or 32 x 64 tiles, a 32 x 32 one the few-tiles kernel (16 or
+ * 32 rows by 16 to 64 columns). */
 int mcke_launch_gemm_f32(const float* a, const float* b, float* c, int64_t m, int64_t n,
                          int64_t k, float alpha, float beta, int variant,
                          const mcke_gemm_tile* tile, void* stream);
@@ -191,7 +194,10 @@ int mcke_launch_gemm_bias_act_f32(const float* a, const float* b, const float* b
                                   int64_t m, int64_t n, int64_t k, float alpha, int activation,
                                   const mcke_gemm_tile* tile, void* stream);
 
-/* gemm_kernel_attrs, kernels.hpp:301-302 / gemm.cu:884-904. */
+/* gemm_kernel_attrs, kernels.hpp:301-302 / gemm.cu:884-904.  For kMfmaF32: the tile's
+ * own kernel for whole tiles and 16-byte aligned operands.  A launch that runs another
+ * kernel of the tile's size class may have another block size (512 lanes for the
+ * few-tiles kernel), LDS footprint and register count. */
 int mcke_gemm_kernel_attrs(int variant, const mcke_gemm_tile* tile,
                            mcke_kernel_attrs* out);
 
@@ -208,18 +214,24 @@ enum mcke_dtype { MCKE_DTYPE_F32 = 0, MCKE_DTYPE_F16 = 1, MCKE_DTYPE_BF16 = 2 };
 
 /* C = alpha * A B + beta * C; A (m x k) and B (k x n) row-major in ab_dtype
  * (MCKE_DTYPE_BF16 or MCKE_DTYPE_F16), products accumulated in fp32
- * (v_mfma_f32_32x32x16_{bf16,f16}), C row-major in c_dtype (MCKE_DTYPE_F32 or
+ * (v_mfma_f32_16x16x32 and 32x32x16), C row-major in c_dtype (MCKE_DTYPE_F32 or
  * ab_dtype, rounded to nearest even).  Validation as mcke_launch_gemm_f32: m or
  * n == 0 is a no-op, k == 0 gives C = beta * C, C is not read when beta == 0,
  * a == c / b == c and negative or > INT32_MAX extents are INVALID_ARGUMENT.
  * Tiles (bm,bn,bk,tm,tn): (256,256,64,16,16), (128,128,64,8,8), (64,64,64,4,4);
- * any other tile is INVALID_ARGUMENT.  Any shape and alignment is accepted;
- * k % 8 == 0, n % 8 == 0 and 16-byte aligned a, b, c take the 16-byte path. */
+ * any other tile is INVALID_ARGUMENT.  Any shape and alignment is accepted.  The
+ * tile names a size class: whole tiles of 256 and 128 (16-byte aligned a, b, c,
+ * k % 64 == 0) run as asked; other shapes run 256 x 256 or 128 x 128 tiles where
+ * there are enough of them to fill the GPU, else a kernel whose waves split k over
+ * tiles of 16 to 64 rows by 32 or 64 columns, as 64 x 64 launches do. */
 int mcke_launch_gemm_lp(const void* a, const void* b, void* c, int ab_dtype, int c_dtype,
                         int64_t m, int64_t n, int64_t k, float alpha, float beta,
                         const mcke_gemm_tile* tile, void* stream);
 
-/* mcke_gemm_kernel_attrs for the whole-tile kernel of one (dtype pair, tile). */
+/* mcke_gemm_kernel_attrs for one (dtype pair, tile): of the kernel that whole tiles of
+ * 256 and 128 run, and of the widest split-k one (64 x 64) for the 64 x 64 tile.
+ * Launches of other shapes may run other kernels, with other block sizes (512 lanes
+ * for up to 32 rows or 63 columns) and LDS footprints. */
 int mcke_gemm_lp_kernel_attrs(int ab_dtype, int c_dtype, const mcke_gemm_tile* tile,
                               mcke_kernel_attrs* out);
 

@@ -554,7 +554,8 @@ def launch_gemm_lp_vendor(a, b, c, ab_dtype, c_dtype, m: int, n: int, k: int, al
 
 
 def gemm_lp_kernel_attrs(ab_dtype, c_dtype, tile: GemmTile):
-    """Returns (Status, KernelAttrs) of the whole-tile kernel."""
+    """Returns (Status, KernelAttrs) of the kernel that whole tiles of 256 and 128 run
+    (for 64 x 64, of the widest split-K kernel)."""
     out = KernelAttrs()
     st = _st(lib().mcke_gemm_lp_kernel_attrs(int(ab_dtype), int(c_dtype), C.byref(tile),
                                              C.byref(out)))
