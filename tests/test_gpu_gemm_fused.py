@@ -5,8 +5,8 @@ Its contract is the pair it replaces: launch_gemm_f32 (kMfmaF32, beta = 0) into 
 then launch_bias_act_f32 on C (the reference's GemmOp -> BiasActOp chain,
 src/graph/ops_gemm.cpp:74-96 and ops_bias_act.cpp:102-130).  So every case here is
 checked bit for bit against that pair on the same tile -- every MFMA tile, whole
-tiles (the direct-to-LDS kernel) and ragged or unaligned shapes (the staged
-kernel), all four activations, several alphas, k = 0 and special values -- and
+tiles, ragged and unaligned shapes (each kernel that a tile's size class may run), all
+four activations, several alphas, k = 0 and special values -- and
 against the CPU oracle (oracle.gemm, then oracle.bias_act on its fp32 result)
 within the GEMM tolerance tol_gemm(k) / abs_tol_gemm(k) plus the bias+act
 tolerance (abs 1e-6 + rel 1e-6), the bars the two launches meet separately."""
@@ -118,6 +118,8 @@ def test_ragged_shapes_match_the_pair(gpu, orc, ti, shape):
 
 @pytest.mark.parametrize("ti", [0, 2, 4, 5], ids=lambda i: f"tile{i}")
 def test_unaligned_operands_take_the_scalar_kernel(gpu, orc, ti):
+    # (80 columns: narrower than the 256 and 128 tiles.  The two small tiles' launches take
+    # the EDGE form of 32 x 64 tiles and the few-tiles kernel at any 4-byte alignment.)
     t = gpu.MFMA_TILES[ti]
     M, N, K = 96, 80, 72
     a, b, bias = _inputs(orc, M, N, K, 11)
@@ -144,8 +146,10 @@ def test_k0_gives_the_activation_of_the_bias(gpu, orc, ti):
 def test_special_values_match_the_pair(gpu, orc):
     """inf and NaN in A and in the bias, and products that overflow: the fused
     epilogue gives NaN and +-inf exactly where the pair does."""
-    for t in (gpu.MFMA_TILES[0], gpu.MFMA_TILES[4], gpu.MFMA_TILES[5]):
-        M, N, K = 2 * t.bm, t.bn, 64
+    T = gpu.MFMA_TILES
+    for t, M, N in [(t, 2 * t.bm, t.bn) for t in (T[0], T[4], T[5])] + \
+            [(T[4], 1024, 1024), (T[5], 512, 544)]:
+        K = 64
         a, b, bias = _inputs(orc, M, N, K, 3)
         a = a.copy()
         bias = bias.copy()

@@ -59,12 +59,12 @@ def _quarters(rng, shape):
     return (rng.integers(-8, 9, size=shape) / 4.0).astype(np.float32)
 
 
-# Whole tiles for the direct-to-LDS kernels (tiles with BN >= 128):
-#   * K % 64 == 32 takes the 32x32x16 kernel; K = 32, 96, 160, 224 give it 1, 3, 5
-#     and 7 K steps of 32 (its 4-stage ring's prologue and tail);
-#   * K % 64 == 0 takes the 16x16x32 kernel, whose ring is 3 steps deep and clamps
-#     the A pair and B step it fetches past the end; K = 64, 128, 192, 320 give it
-#     2, 4, 6 and 10 steps (K = 64: fewer steps than the ring is deep).
+# Whole tiles of 256 and 128:
+#   * K % 64 == 0 takes the direct-to-LDS 16x16x32 kernel, whose ring is 3 steps deep and
+#     clamps the A pair and B step it fetches past the end; K = 64, 128, 192, 320 give it
+#     2, 4, 6 and 10 steps (K = 64: fewer steps than the ring is deep);
+#   * K % 64 == 32, at so few tiles, takes the split-K kernel (K = 32, 96, 160, 224: 1, 3, 5
+#     and 7 chunks), as 64 x 64 tiles and the ragged shapes from 32 columns up do.
 QSHAPES = [(1, 1, 1), (5, 7, 3), (129, 65, 257), (1, 64, 128), (64, 1, 128), (33, 63, 1),
            (253, 253, 253), (256, 256, 256), (512, 512, 512),
            (256, 256, 32), (256, 256, 96), (256, 512, 160), (512, 256, 224),
@@ -117,8 +117,8 @@ def test_random_within_gemm_tolerance(gpu, orc, dt, out, shape):
 
 @pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
 def test_unaligned_and_ragged_take_the_element_path_with_same_bits(gpu, orc, dt):
-    # K % 8 != 0 or a misaligned base forces per-element loads; the MFMA sequence
-    # is the same, so the bits match the 16-byte path where both apply.
+    # The split-K kernel loads 16 bytes at any 2-byte alignment: the same bits for an
+    # aligned base and a shifted one.
     M, N, K = 200, 136, 264
     a16 = orc.to_16(orc.fill_random(M * K, 11), dt)
     b16 = orc.to_16(orc.fill_random(K * N, 12), dt)
@@ -240,7 +240,8 @@ def test_kernel_attrs(gpu):
                 # (bm x 128 bytes) and four B steps of 32 k (32 x bn x 2 bytes).
                 assert at.static_smem_bytes == 3 * tile.bm * 128 + 4 * 32 * tile.bn * 2
             else:
-                assert at.static_smem_bytes == 2 * (tile.bm + tile.bn) * 128
+                # Split-K kernel: a slot of 32 k for each of four waves.
+                assert at.static_smem_bytes == 4 * (tile.bm + tile.bn) * 64
             assert at.threads_per_block == 256 and at.max_blocks_per_sm_api >= 1
 
 

@@ -24,6 +24,9 @@ EDGE_128 = [(1279, 1024, 64), (1151, 1150, 66), (1025, 1154, 94), (10200, 130, 1
             (129, 10112, 126), (1663, 2048, 64), (1919, 1790, 66), (1665, 2050, 94),
             (10200, 330, 160), (129, 13440, 126), (1151, 1150, 290)]
 EDGE_256 = [(3073, 4000, 66), (3100, 4098, 128)]
+# Whole 128 x 128 tiles, 80 of them or more, with K % 64 == 32: the direct-to-LDS 32x32x16
+# kernel, 1, 3, 5 and 7 K steps of 32 (its 4-stage ring's prologue and tail).
+DMA_32 = [(1280, 1024, 32), (1280, 1024, 96), (1152, 1280, 160), (1024, 1280, 224)]
 # The register-staged kernel's WHOLE form: odd N or K, from 208 tiles of 128 or 192 of 256
 # on; K % 64 of 0, 1, 32, 63 as the first stage, one and two stages, last tile columns of 1
 # and 127 columns of their own.
@@ -93,6 +96,14 @@ def test_edge_tiles(gpu, orc, dt, out, shape):
     tile = gpu.LP_TILES[0] if shape in EDGE_256 else gpu.LP_TILES[1]
     _check(gpu, orc, dt, out, *shape, tile, (0, 0, 0), 1.0, 0.0)
     _check(gpu, orc, dt, out, *shape, tile, (2, 4, 2), 0.5, 2.0)
+
+
+@pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
+@pytest.mark.parametrize("out", ["f32", "same"])
+@pytest.mark.parametrize("shape", DMA_32, ids=lambda s: "x".join(map(str, s)))
+def test_whole_tiles_of_32_deep_stages(gpu, orc, dt, out, shape):
+    _check(gpu, orc, dt, out, *shape, gpu.LP_TILES[1], (0, 0, 0), 1.0, 0.0)
+    _check(gpu, orc, dt, out, *shape, gpu.LP_TILES[1], (0, 0, 0), 0.5, 2.0)
 
 
 @pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)

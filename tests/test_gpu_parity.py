@@ -509,10 +509,9 @@ def test_gemm_dma_ring_step_counts(gpu, orc, tile, mnk):
 @pytest.mark.parametrize("tile", [(64, 64, 32, 4, 4), (32, 32, 32, 2, 2)])
 @pytest.mark.parametrize("n", [32, 64, 192, 512, 1024, 100, 257])
 def test_gemm_wave_group_tiles(gpu, orc, tile, n):
-    """The small tiles' size classes: 64x64 (whole tiles of 64x64 at n = 1024, 32x64
-    tiles below) and 32x32 (the few-tiles kernel, whose eight waves split K, up to n =
-    257 and past that at n = 512 and 1024 the tile's four wave groups, folded in a fixed
-    order): the full reference (reference.hpp:199-211) at the
+    """The small tiles' size classes: 64x64 (its own tiles at n = 1024, 32x64 ones from
+    64 to 512) and 32x32 (the few-tiles kernel, whose eight waves split K, at n = 64, 100
+    and 192, else the tile's four wave groups, folded in a fixed order): the full reference (reference.hpp:199-211) at the
     K-scaled tolerance, the same bits on a second launch, and beta = 0 never
     reading a NaN-poisoned C."""
     a = orc.fill_random(n * n, 0x6E33A + n)
