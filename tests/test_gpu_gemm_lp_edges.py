@@ -132,6 +132,18 @@ def test_short_k(gpu, orc, dt, out, shape):
     _check(gpu, orc, dt, out, *shape, tile, (1, 3, 1), 0.5, 2.0)
 
 
+@pytest.mark.parametrize("dt", DTS, ids=DT_ID.get)
+@pytest.mark.parametrize("out", ["f32", "same"])
+@pytest.mark.parametrize("shape", [(300, 24, 72), (70, 8, 128), (513, 16, 8)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_narrow_products_on_every_tile(gpu, orc, dt, out, shape):
+    """Below 32 columns: the register-staged kernel at the requested tile, 16 bytes a load
+    and element by element."""
+    for tile in gpu.LP_TILES:
+        _check(gpu, orc, dt, out, *shape, tile, (0, 0, 0), 1.0, 0.0)
+        _check(gpu, orc, dt, out, *shape, tile, (1, 3, 1), 0.5, 2.0)
+
+
 def test_remainders_keep_special_values_apart(gpu, orc):
     """The K remainder pads both operands with zeros: infinities and NaN in the last columns
     of A and the last rows of B reach their own outputs only."""

@@ -6,7 +6,8 @@ Every output buffer has guard floats around it that must keep their bits.
 Bars: softmax rel 1e-5 + abs 1e-6 (the fixed-shape tests' bar); max exact; sums in
 float64 within 2^-24 times the longest chain of adds a lane and its combine can make
 (cols / 32 + 16 at most for these layouts), relative to the row's sum of magnitudes;
-bias + activation bit-equal to the capped launch, which walks rows with the row kernel.
+bias + activation bit-equal to the capped launch, which walks rows in chunks, and past 4096
+workgroups with the row kernel; there also against the oracle at abs 1e-6 + rel 1e-6.
 """
 from __future__ import annotations
 
@@ -46,7 +47,8 @@ def _up(m, x, shift):
 # (x, y) offsets in floats; GUARD is a multiple of 4, so (0, 0) is the aligned one.
 SHIFTS = [(0, 0), (1, 1), (3, 2), (0, 3)]
 SOFTMAX_COLS = [1, 2, 3, 5, 35, 36, 39, 67, 68, 71, 131, 259, 260, 263, 515, 519, 1027, 1031,
-                2055, 4103, 8195, 8200, 16387, 16391, 32771, 32776, 65536, 65539, 65540, 65543]
+                2055, 4103, 8195, 8200, 16387, 16391, 32768, 32771,
+                32776, 65536, 65539, 65540, 65543]
 
 
 @pytest.mark.parametrize("cols", SOFTMAX_COLS)
@@ -157,3 +159,31 @@ def test_bias_act_any_width_matches_the_row_kernel(gpu, orc, cols, act):
         gpu.device_synchronize()
         assert np.array_equal(out.get().view(np.uint32), want), f"shift={sx},{sy},{sb}"
     del db, dx
+
+
+@pytest.mark.parametrize("act", [0, 1, 2, 3])
+@pytest.mark.parametrize("cols", [100, 256])
+def test_bias_act_kernels_of_many_rows_agree(gpu, orc, cols, act):
+    """4101 rows: capped launches walk them with the row kernel (7 workgroup rows, and one
+    per row), the others run as one flat array or, at vw = 4 and 256 columns, as whole 1 KiB
+    strips."""
+    rows = 4101
+    x = orc.fill_normal(rows * cols, 0xB1A7 + cols, 0.0, 2.0)
+    bias = orc.fill_random(cols, 0xB1A8 + cols, -0.5, 0.5)
+    want = orc.bias_act(x, bias, rows, cols, act)
+    dx, px = _up(gpu, x, 0)
+    db, pb = _up(gpu, bias, 0)
+    seen = None
+    for vw in (1, 2, 4):
+        for cap in (7, rows, 0):
+            out = _Out(gpu, rows * cols, 0)
+            st = gpu.launch_bias_act_f32(px, pb, out.ptr, rows, cols, act, vw, None, cap)
+            assert st.ok(), str(st)
+            gpu.device_synchronize()
+            got = out.get()
+            if seen is None:
+                seen = got.view(np.uint32).copy()
+                r = orc.compare(got, want, 1e-6, 1e-6)
+                assert r.ok, str(r)
+            assert np.array_equal(got.view(np.uint32), seen), f"vw={vw} cap={cap}"
+    del dx, db
