@@ -31,7 +31,7 @@ def _nan_aware_bits_equal(got, want):
 
 def _run(m, a, b, bias, M, N, K, alpha, act, tile, offset=0):
     """Fused and unfused outputs on the same device inputs.  `offset` floats
-    shift every operand off 16-byte alignment (the staged scalar kernel)."""
+    shift every operand off 16-byte alignment."""
     D = m.DeviceBuffer
 
     def up(arr, n):

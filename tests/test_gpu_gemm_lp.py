@@ -143,7 +143,7 @@ def test_unaligned_and_ragged_take_the_element_path_with_same_bits(gpu, orc, dt)
 @pytest.mark.parametrize("out", ["f32", "same"])
 @pytest.mark.parametrize("shape", [(67, 45, 39), (256, 256, 64)], ids=lambda s: "x".join(map(str, s)))
 def test_special_values(gpu, orc, dt, out, shape):
-    """16-bit infinities and NaN in A and B, every tile, ragged (element path) and
+    """16-bit infinities and NaN in A and B, every tile, ragged (split-K kernel) and
     whole-tile (direct-to-LDS kernel) shapes: NaN and +-inf in C exactly where the
     oracle has them (no summation order changes those), finite entries within
     tol_gemm(k) plus one output ulp for 16-bit C."""

@@ -206,7 +206,7 @@ def test_row_reduce_random(gpu, orc, variant, shape):
             assert r.ok, f"kind={kind}: {r}"
 
 
-@pytest.mark.parametrize("cols", [5, 1000, 70000])
+@pytest.mark.parametrize("cols", [5, 1000, 1031, 70000])
 def test_row_reduce_special_values(gpu, orc, cols):
     """Sum, max and mean of rows holding +inf, -inf, both, NaN, or huge values, every
     variant: the same NaN / +-inf pattern as the double-precision reference
@@ -264,15 +264,16 @@ def test_softmax_random(gpu, orc, variant, cols):
     assert np.max(np.abs(sums - 1.0)) <= 1e-5
 
 
-@pytest.mark.parametrize("cols", [7, 8, 1024, 1031, 8200])
+@pytest.mark.parametrize("cols", [7, 8, 259, 1024, 1031, 8200, 32771, 65543, 65548])
 def test_softmax_special_values(gpu, orc, cols):
     """Rows with infinities, NaN, huge and tiny magnitudes against the double-precision
     reference (reference.hpp:175-191): its max keeps the running value against NaN
     (std::max(m, v)), so a NaN entry, a +inf entry or a row of -inf makes the whole
     row NaN through the sum, while -inf and -FLT_MAX entries beside finite ones get 0.
-    Every kernel path: cols 7 and 1031 take the element path, 8 and 1024 the
-    register-resident kernel, 8200 the one-pass online kernel on 16-byte data; both
-    variants.  NaN positions must match; other entries rel 1e-5 + abs 1e-6."""
+    Every kernel path: the register-resident kernel with edge elements (odd cols) and
+    without, in a wave and over several, up to 16 float4s a lane (32771), and past 65539
+    columns the one-pass online kernel; both variants.  NaN positions must match; other
+    entries rel 1e-5 + abs 1e-6."""
     fmax = np.finfo(np.float32).max
     rng = np.random.default_rng(cols)
     rows = []
