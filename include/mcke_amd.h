@@ -223,7 +223,8 @@ enum mcke_dtype { MCKE_DTYPE_F32 = 0, MCKE_DTYPE_F16 = 1, MCKE_DTYPE_BF16 = 2 };
  * tile names a size class: whole tiles of 256 and 128 (16-byte aligned a, b, c,
  * k % 64 == 0) run as asked; other shapes run 256 x 256 or 128 x 128 tiles where
  * there are enough of them to fill the GPU, else a kernel whose waves split k over
- * tiles of 16 to 64 rows by 32 or 64 columns, as 64 x 64 launches do. */
+ * tiles of 16 to 64 rows by 32 or 64 columns, as 64 x 64 launches do, or for short k
+ * over many tiles and less than 32 columns a register-staged one. */
 int mcke_launch_gemm_lp(const void* a, const void* b, void* c, int ab_dtype, int c_dtype,
                         int64_t m, int64_t n, int64_t k, float alpha, float beta,
                         const mcke_gemm_tile* tile, void* stream);

@@ -181,7 +181,7 @@ struct LpTile {
   // 22.1; 3001 x 2501 x 901, 480 tiles, 33.1 against 50.0), at 256 x 256 from 192 such tiles on
   // (4095^3 199 us against 229 at 128 and 406 for split K; 3500 x 3501 x 2001, 196 tiles, 99
   // against 105).  What is left takes the split-K kernel, as 64 x 64 launches do, but for
-  // short K over many tiles (short_k).
+  // short K over many tiles (short_k).  The tile counts here and below are for 256 CUs.
   static int launch(const LpArgs& x, bool vec) {
     if constexpr (BN >= 128) {
       if (vec && x.m % BM == 0 && x.n % BN == 0 && x.k % 64 == 0 && x.k > 0 &&

@@ -1,7 +1,7 @@
 // gemm_lp.hpp -- 16-bit-input GEMM on the CDNA4 matrix cores, fp32 accumulation.
 // Kernels: gemm_lp_kernel (any shape, register-staged, 32x32x16 MFMAs, the layout
-// described first below; large products of odd extents and those narrower than 32 columns
-// take it),
+// described first below; large products of odd extents or short K and those narrower than
+// 32 columns take it),
 // gemm_lp_dma_kernel (direct-to-LDS, 32x32x16; whole 128 x 128 tiles with K % 64 == 32),
 // gemm_lp_dma16_kernel (direct-to-LDS, 16x16x32; whole tiles with K % 64 == 0, and an
 // EDGE form for other even shapes), each described where it is defined, and
