@@ -807,16 +807,11 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma_kernel(
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         Quad* dst = reinterpret_cast<Quad*>(crow + 32 * j + 8 * g);
+        const Quad old = *dst;
         Quad o;
-        if (beta != 0.0f) {
-          const Quad old = *dst;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            o.v[e] = O::from_f32(alpha * acc[i][j][4 * g + e] + beta * O::to_f32(old.v[e]));
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o.v[e] = O::from_f32(alpha * acc[i][j][4 * g + e]);
-        }
+        for (int e = 0; e < 4; ++e)
+          o.v[e] = O::from_f32(alpha * acc[i][j][4 * g + e] + beta * O::to_f32(old.v[e]));
         *dst = o;
       }
     }
