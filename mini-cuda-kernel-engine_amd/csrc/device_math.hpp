@@ -15,6 +15,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // dword alignment).
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
+// Steps of `step` that cover `extent`, which goes up to INT32_MAX: extent + step - 1 does
+// not fit an int there.
+__host__ __device__ constexpr int steps_along(int extent, int step) {
+  return extent / step + (extent % step != 0 ? 1 : 0);
+}
+static_assert(steps_along(INT32_MAX, 256) == 1 << 23 && steps_along(INT32_MAX, 8) == 1 << 28 &&
+              steps_along(64, 64) == 1 && steps_along(1, 64) == 1 && steps_along(0, 64) == 0);
+
 template <int VW> struct VecT;
 template <> struct VecT<1> { using type = float; };
 template <> struct VecT<2> { using type = f32x2; };

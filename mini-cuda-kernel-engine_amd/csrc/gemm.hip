@@ -62,7 +62,8 @@ __global__ __launch_bounds__(1024) void gemm_tiled_smem_kernel(const float* __re
   const int tx = threadIdx.x, ty = threadIdx.y;
   const int row = blockIdx.y * T + ty, col = blockIdx.x * T + tx;
   float acc = 0.0f;
-  for (int k0 = 0; k0 < k; k0 += T) {
+  for (int kt = 0; kt < steps_along(k, T); ++kt) {
+    const int k0 = kt * T;
     As[ty][tx] = (row < m && k0 + tx < k) ? a[static_cast<int64_t>(row) * k + k0 + tx] : 0.0f;
     Bs[ty][tx] = (k0 + ty < k && col < n) ? b[static_cast<int64_t>(k0 + ty) * n + col] : 0.0f;
     __syncthreads();
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(256) void gemm_regblock_kernel(const float* __restr
     }
   };
 
-  const int ktiles = (k + BK - 1) / BK;
+  const int ktiles = steps_along(k, BK);
   if (DBUF) {
     if (ktiles > 0) {
       gload(0);

@@ -27,15 +27,8 @@ bool dma_offsets32(int n, int k) {
          static_cast<int64_t>(64) * n * 2 < (int64_t{1} << 32);
 }
 
-// Tiles along one extent.  Extents go up to INT32_MAX, where extent + tile - 1 does not fit
-// an int.
-constexpr int tiles_along(int extent, int tile) {
-  return static_cast<int>((static_cast<int64_t>(extent) + tile - 1) / tile);
-}
-static_assert(tiles_along(INT32_MAX, 256) == 1 << 23 && tiles_along(1, 256) == 1);
-
 int64_t tile_count(int m, int n, int bm, int bn) {
-  return static_cast<int64_t>(tiles_along(m, bm)) * tiles_along(n, bn);
+  return static_cast<int64_t>(steps_along(m, bm)) * steps_along(n, bn);
 }
 
 struct LpArgs {
@@ -61,7 +54,7 @@ int launch_dma(const LpArgs& x) {
   gemm_lp_dma16_kernel<T, OutT, BM, BN, EDGE>
       <<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
           x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
-          tiles_along(x.m, BM), tiles_along(x.n, BN));
+          steps_along(x.m, BM), steps_along(x.n, BN));
   MCKE_LAUNCH_CHECK("gemm_lp_dma16_kernel");
   return ok();
 }
@@ -74,7 +67,7 @@ int launch_split_as(const LpArgs& x) {
   gemm_lp_split_kernel<T, OutT, MT, NW, WV>
       <<<static_cast<unsigned>(tiles), WV * kWave, 0, x.s>>>(
           x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
-          tiles_along(x.m, TM), tiles_along(x.n, TN));
+          steps_along(x.m, TM), steps_along(x.n, TN));
   MCKE_LAUNCH_CHECK("gemm_lp_split_kernel");
   return ok();
 }
@@ -103,7 +96,7 @@ int launch_staged(const LpArgs& x, bool vec) {
                  : &gemm_lp_kernel<T, OutT, BM, BN, false, false>;
   fn<<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
       x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
-      tiles_along(x.m, BM), tiles_along(x.n, BN));
+      steps_along(x.m, BM), steps_along(x.n, BN));
   MCKE_LAUNCH_CHECK("gemm_lp_kernel");
   return ok();
 }
@@ -135,7 +128,7 @@ int launch_whole(const LpArgs& x) {
   gemm_lp_kernel<T, OutT, BM, BN, false, true>
       <<<static_cast<unsigned>(tiles), kMfmaThreads, 0, x.s>>>(
           x.a, x.b, static_cast<OutT*>(x.c), x.m, x.n, x.k, x.alpha, x.beta,
-          tiles_along(x.m, BM), tiles_along(x.n, BN));
+          steps_along(x.m, BM), steps_along(x.n, BN));
   MCKE_LAUNCH_CHECK("gemm_lp_kernel");
   return ok();
 }

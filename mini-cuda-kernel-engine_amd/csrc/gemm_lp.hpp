@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int ksteps = (K + kLpBK - 1) / kLpBK;
+  const int ksteps = steps_along(K, kLpBK);
   // Stage s > 0 starts at k = 64 s - k_short.
   const int rem = WHOLE ? K % kLpBK : 0;
   const int k_short = rem ? kLpBK - rem : 0;
@@ -1141,7 +1141,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_lp_dma16_kernel(
 
   const uint32_t lds0 = lds_addr(smem);
   const uint32_t ldsb = lds0 + S::kBBase;
-  const int ksteps = EDGE ? 2 * ((K + 63) / 64) : K / BK;   // even
+  const int ksteps = EDGE ? 2 * steps_along(K, 64) : K / BK;   // even
   const int last_pair = ksteps / 2 - 1;
   u32x4 av[2][MT];
   u32x2 bv[2][NT][2];

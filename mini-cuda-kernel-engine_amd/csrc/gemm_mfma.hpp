@@ -629,7 +629,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void gemm_mfma_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int ksteps = (K + BK - 1) / BK;
+  const int ksteps = steps_along(K, BK);
   typename S::Regs R;
   if (ksteps > 0) {
     S::load(R, A, B, M, N, K, m0, n0, 0);
@@ -911,7 +911,7 @@ __global__ __launch_bounds__((kDmaThreads<BM, BN, KS>), 1) void gemm_mfma_dma_ke
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int ksteps = EDGE ? (K + BK - 1) / BK : K / BK;
+  const int ksteps = EDGE ? steps_along(K, BK) : K / BK;
   // Prologue: stages 0 .. STAGES-2 in flight.  Past the last K step a stage
   // re-fetches the last one into a buffer nobody reads, which keeps the number of
   // loads per stage -- and so the vmcnt arithmetic below -- uniform.
