@@ -16,7 +16,7 @@
 //                row folds that row's partials in a fixed order (a second
 //                launch, as reduce.cu:180-206).  Rows that need no split are
 //                written out by the first launch, which is then the only one (up to
-//                1027 columns it is kWarpShuffle's).
+//                2051 columns it is kWarpShuffle's).
 //                With rows == 1 this is the full-tensor reduction.
 // Every variant is deterministic (nothing is combined atomically) and keeps no
 // state between launches: the same input gives the same bits on every run, on
@@ -262,8 +262,11 @@ int64_t two_pass_split(int64_t rows, int64_t cols) {
   return s;
 }
 
-// The longest rows, in float4s, that lanes of one wave own (launch_one_pass).
+// The longest rows, in float4s, that lanes of one wave own (launch_one_pass), and that
+// kTwoPass leaves to the one-pass kernels.
 constexpr int64_t kShortVectors = 256;
+constexpr int64_t kOnePassVectors = 512;
+static_assert(4 * kOnePassVectors + 3 < 2 * kMinColsPerBlock, "rows that are never split");
 
 template <class Op, bool MEAN, int TPR>
 int launch_short(const float* x, float* out, int64_t rows, int64_t cols, bool aligned16,
@@ -310,8 +313,10 @@ template <class Op, bool MEAN>
 int launch_two_pass(const float* x, float* out, int64_t rows, int64_t cols, float* part,
                     hipStream_t st) {
   // Short rows are never split, and a 512-lane workgroup per row costs more than their loads:
-  // the one-pass kernel for them (41109 x 82: 4.4 us for 59.3; 22016 x 726: 10.7 for 37.1).
-  if (cols / 4 <= kShortVectors) return launch_one_pass<Op, MEAN>(x, out, rows, cols, false, st);
+  // the one-pass kernels (41109 x 82: 4.4 us for 59.3; 22016 x 726: 10.7 for 37.1; 10613 x
+  // 1452: 10.3 for 16.7; 2914 x 1954: 5.4 for 6.75).  They lead less and less up to 4096
+  // columns (3076 x 3644: 8.4 for 8.5) and trail past that (2287 x 4380: 8.05 for 7.6).
+  if (cols / 4 <= kOnePassVectors) return launch_one_pass<Op, MEAN>(x, out, rows, cols, false, st);
   const int64_t split = two_pass_split(rows, cols);
   // chunk is a multiple of 4 so each chunk keeps the row's 16-byte alignment.
   int64_t chunk = (cols + split - 1) / split;

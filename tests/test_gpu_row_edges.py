@@ -69,7 +69,7 @@ def test_softmax_width_edges(gpu, orc, cols):
 
 
 REDUCE_COLS = [1, 2, 5, 7, 31, 128, 131, 132, 133, 256, 259, 260, 263, 515, 516, 519, 1027, 1028,
-               1031, 4095, 4099]
+               1031, 2048, 2051, 2052, 2055, 4095, 4099]
 
 
 @pytest.mark.parametrize("cols", REDUCE_COLS)
